@@ -231,7 +231,9 @@ uint32_t maize_hip_get_split_wait_us(void);
  * fails with MAIZE_ERR_KERNEL if that kernel cannot run the descriptor. */
 int32_t maize_hip_gemm_bf16_with(maize_ctx_t* ctx, const maize_gemm_desc_t* desc,
                                  const char* kernel, void* stream);
-/* Which kernel maize_hip_gemm_bf16 would pick; writes a NUL-terminated name. */
+/* Which kernel maize_hip_gemm_bf16 would pick; writes a NUL-terminated name.  (What this and maize_hip_gemm_plan report is the
+ * registry's choice.  Where no kernel is named the launcher may run one of its own forms in its place -- small tiles for any
+ * alignment, maize_amd/csrc/forms.hpp -- with the same operand handling and accuracy.  Naming the kernel runs exactly it.) */
 int32_t maize_hip_gemm_select(maize_ctx_t* ctx, const maize_gemm_desc_t* desc, char* name, size_t cap);
 /* Launch geometry for `desc` on a device with `compute_units` compute units (no device access):
  * which kernel (`kernel` == NULL: the dispatcher's choice), its grid and block, the number of K

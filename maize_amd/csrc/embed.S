@@ -1,4 +1,4 @@
-/* Embeds the gfx950 code object into libmaize_hip.so. */
+/* Embeds the gfx950 code objects into libmaize_hip.so. */
     .section .rodata
     .balign 4096
     .global maize_embedded_hsaco
@@ -10,4 +10,12 @@ maize_embedded_hsaco:
 maize_embedded_hsaco_end:
     .byte 0
     .size maize_embedded_hsaco, maize_embedded_hsaco_end - maize_embedded_hsaco
+    .balign 4096
+    .global maize_embedded_forms
+    .type maize_embedded_forms, @object
+maize_embedded_forms:
+    .incbin MAIZE_FORMS_PATH
+    .byte 0
+    .size maize_embedded_forms, . - maize_embedded_forms
+
     .section .note.GNU-stack,"",@progbits

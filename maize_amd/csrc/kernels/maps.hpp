@@ -100,6 +100,20 @@ MAIZE_MAP uint32_t sk128_tr_offset(uint32_t cg, uint32_t h, uint32_t lane) {
     return sk128_offset(sk_tr_row(h, lane), col >> 3) + (col & 7u) * 2u;
 }
 
+// ---- K x N operand tile 64 columns wide (row-major B): 64 rows of 128 B, 8 pieces --------------------------------
+// Piece p (8 rows, 1 KiB): lane l lands at row 8p + l/8, position l%8.  Rows of one parity share 32 banks, so the four
+// 32-byte granules of a row are XOR-ed with f(row) = bit1(row) + 2 bit3(row), which tells the four rows of a parity apart
+// that a 32-lane pass of a transposing read touches (row%4 and bit 3 vary).  K half kh and register half h of a read sit
+// 4096 kh + 512 h bytes behind (0, 0).
+MAIZE_MAP uint32_t sk64_swizzle(uint32_t row) { return ((row >> 1) & 1u) | (((row >> 3) & 1u) << 1); }
+MAIZE_MAP uint32_t sk64_piece_row(uint32_t piece, uint32_t lane) { return piece * 8u + (lane >> 3); }
+MAIZE_MAP uint32_t sk64_piece_chunk(uint32_t piece, uint32_t lane) { return (lane & 7u) ^ (sk64_swizzle(sk64_piece_row(piece, lane)) << 1); }
+MAIZE_MAP uint32_t sk64_offset(uint32_t row, uint32_t chunk) { return row * 128u + ((chunk ^ (sk64_swizzle(row) << 1)) * 16u); }
+MAIZE_MAP uint32_t sk64_tr_offset(uint32_t cg, uint32_t h, uint32_t lane) {
+    const uint32_t col = cg * 16u + (lane & 3u) * 4u;
+    return sk64_offset(sk_tr_row(h, lane), col >> 3) + (col & 7u) * 2u;
+}
+
 // ---- The ragged last columns of a K x N / N x K B riding along in the macro-tile K loop: a 64 x 16 tile (2 KiB) ----
 // Brought in by 4-byte-per-lane requests of 256 bytes, two per wave (request q = 2 wave + j, 0..7), landing linearly.
 // K x N: 64 rows of 32 bytes (columns 0..15), no swizzle; request q covers rows 8 q .. + 7: lane l fetches row
@@ -145,6 +159,17 @@ MAIZE_MAP uint32_t sk8n_offset(uint32_t row, uint32_t chunk) { return row * 128u
 // Transposing read (ds_read_b64_tr_b8) as for the wide tile: read (kk, h) of column group cg fetches rows 64 kk + 16 g + 8 h + 0..7.
 MAIZE_MAP uint32_t sk8n_tr_offset(uint32_t cg, uint32_t kk, uint32_t h, uint32_t lane) {
     return sk8n_offset(sk8_tr_row(kk, h, lane), cg) + (lane & 1u) * 8u;
+}
+
+// ---- K x N operand tile of 8-bit elements, 64 columns wide: 128 rows of 64 B, 8 pieces ----------------------------
+// Piece p (16 rows, 1 KiB): lane l lands at row 16p + l/4, position l%4.  Rows equal mod 4 share 16 banks: the chunk index is
+// XOR-ed with f(row) = bit2(row) + 2 bit4(row).  The four reads of a fragment sit 512 (8 rows) and 4096 (64 rows) bytes apart.
+MAIZE_MAP uint32_t sk8s_swizzle(uint32_t row) { return ((row >> 2) & 1u) | (((row >> 4) & 1u) << 1); }
+MAIZE_MAP uint32_t sk8s_piece_row(uint32_t piece, uint32_t lane) { return piece * 16u + (lane >> 2); }
+MAIZE_MAP uint32_t sk8s_piece_chunk(uint32_t piece, uint32_t lane) { return (lane & 3u) ^ sk8s_swizzle(sk8s_piece_row(piece, lane)); }
+MAIZE_MAP uint32_t sk8s_offset(uint32_t row, uint32_t chunk) { return row * 64u + ((chunk ^ sk8s_swizzle(row)) * 16u); }
+MAIZE_MAP uint32_t sk8s_tr_offset(uint32_t cg, uint32_t kk, uint32_t h, uint32_t lane) {
+    return sk8s_offset(sk8_tr_row(kk, h, lane), cg) + (lane & 1u) * 8u;
 }
 
 }  // namespace maps

@@ -15,10 +15,12 @@
 #include <unordered_map>
 
 #include "dispatch.hpp"
+#include "forms.hpp"
 #include "noalloc.hpp"
 
 extern "C" const unsigned char maize_embedded_hsaco[];
 extern "C" const unsigned char maize_embedded_hsaco_end[];
+extern "C" const unsigned char maize_embedded_forms[];       // the launcher's own forms (forms.hpp)
 
 static_assert(sizeof(maize_matrix_t) == 16 && alignof(maize_matrix_t) == 16, "GlobalMatrix twin");
 static_assert(sizeof(maize_gemm_args_t) == 120, "kernel parameter block");
@@ -80,6 +82,8 @@ struct maize_ctx {
     hipDeviceProp_t prop;
     hipModule_t module;
     hipFunction_t fn[maize::kMaxKernels];
+    hipModule_t forms_module;
+    hipFunction_t form_fn[maize::kMaxForms];
     hipFunction_t reduce_fn;
     hipFunction_t pack_fn, pack_u8_fn, transpose_u8_fn;
     // Split-K scratch, one per stream so that launches on different streams never share it.
@@ -161,6 +165,25 @@ int32_t maize_hip_ctx_create(int32_t device, maize_ctx_t** out) {
         delete ctx;
         return rc;
     }
+    e = hipModuleLoadData(&ctx->forms_module, maize_embedded_forms);
+    if (e != hipSuccess) {
+        int32_t rc = hip_fail(e, "hipModuleLoadData(embedded code object of the launcher's forms)");
+        (void)hipModuleUnload(ctx->module);
+        delete ctx;
+        return rc;
+    }
+    for (uint32_t i = 0; i < maize::form_count(); ++i) {
+        const char* name = maize::form_name(i);
+        if (!name) continue;
+        e = hipModuleGetFunction(&ctx->form_fn[i], ctx->forms_module, name);
+        if (e != hipSuccess) {
+            int32_t rc = hip_fail(e, name);
+            (void)hipModuleUnload(ctx->forms_module);
+            (void)hipModuleUnload(ctx->module);
+            delete ctx;
+            return rc;
+        }
+    }
     // The device is current here: look up the address of its copy of the no-allocation scratch array.  A failure
     // only disables maize_hip_gemm_bf16_noalloc (which then reports it).
     ctx->scratch_err = maize::noalloc_scratch(device, &ctx->scratch.ptr, &ctx->scratch.bytes);
@@ -175,6 +198,8 @@ int32_t maize_hip_ctx_destroy(maize_ctx_t* ctx) {
     for (auto& kv : ctx->workspaces)
         if (kv.second.ptr) (void)hipFree(kv.second.ptr);
     hipError_t e = hipModuleUnload(ctx->module);
+    const hipError_t ef = hipModuleUnload(ctx->forms_module);
+    if (e == hipSuccess) e = ef;
     delete ctx;
     if (e != hipSuccess) return hip_fail(e, "hipModuleUnload");
     return MAIZE_OK;
@@ -452,11 +477,8 @@ static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void*
     return MAIZE_OK;
 }
 
-// `fixed`: NULL = the stream's own workspace (allocated or grown here); else the caller's fixed scratch memory, which
-// is used as it is and never grown (a launch that needs more fails).
-static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint32_t idx, void* stream,
-                           const maize_workspace* fixed = nullptr) {
-    const maize::KernelInfo& ki = maize::kernel_at(idx);
+// The kernel parameter block of a descriptor, without what a plan adds (workspace, K ranges, launch flags).
+static maize_gemm_args_t args_of(const maize_gemm_ex_desc_t* x) {
     const maize_gemm_desc_t* d = &x->gemm;
     maize_gemm_args_t args;
     memset(&args, 0, sizeof args);
@@ -474,6 +496,16 @@ static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint
                (x->in_type == MAIZE_IN_F16 ? 4u : 0u) | (x->out_type == MAIZE_OUT_F16 ? 64u : 0u) | ((x->in_type >= MAIZE_IN_E4M3 && x->in_type <= MAIZE_IN_E5M2_E4M3) ? 8u : 0u) |
                ((x->in_type == MAIZE_IN_E5M2 || x->in_type == MAIZE_IN_E5M2_E4M3) ? 16u : 0u) |       // A is E5M2
                ((x->in_type == MAIZE_IN_E5M2 || x->in_type == MAIZE_IN_E4M3_E5M2) ? 32u : 0u);        // B is E5M2
+    return args;
+}
+
+// `fixed`: NULL = the stream's own workspace (allocated or grown here); else the caller's fixed scratch memory, which
+// is used as it is and never grown (a launch that needs more fails).
+static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint32_t idx, void* stream,
+                           const maize_workspace* fixed = nullptr) {
+    const maize::KernelInfo& ki = maize::kernel_at(idx);
+    const maize_gemm_desc_t* d = &x->gemm;
+    maize_gemm_args_t args = args_of(x);
     maize::LaunchDims ld;
     memset(&ld, 0, sizeof ld);
     if (!ki.plan(*x, (uint32_t)ctx->prop.multiProcessorCount, &ld))
@@ -537,6 +569,29 @@ static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint
                       sizeof args);
 }
 
+// Runs one of the launcher's own forms.  *ran = false: it cannot be run here (its workspace would have to be allocated while
+// the stream is being captured, which the registry kernel may not need): nothing was launched.
+static int32_t form_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, const maize::FormPlan& f, void* stream,
+                           const maize_workspace* fixed, bool* ran) {
+    maize_gemm_args_t args = args_of(x);
+    args.ksplit = f.ksplit;
+    *ran = false;
+    if (f.workspace_bytes && fixed) {
+        if (f.workspace_bytes > fixed->bytes) return MAIZE_OK;
+        args.workspace = fixed->ptr;
+    } else if (f.workspace_bytes) {
+        if (ctx->workspaces[stream].bytes < f.workspace_bytes) {
+            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return MAIZE_OK;
+        }
+        int32_t rc = workspace_for(ctx, stream, f.workspace_bytes, &args.workspace);
+        if (rc != MAIZE_OK) return rc;
+    }
+    *ran = true;
+    const uint32_t grid[3] = {f.grid, 1, 1}, block[3] = {256, 1, 1};
+    return launch_raw(ctx->device, (uint32_t)ctx->prop.sharedMemPerBlock, ctx->form_fn[f.kernel], grid, block, 0, stream, &args, sizeof args);
+}
+
 // Whether the plan of kernel `idx` for `x` fits the caller's fixed scratch memory; nothing is launched.
 static int32_t fits_fixed(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint32_t idx, const maize_workspace* fixed) {
     const maize::KernelInfo& ki = maize::kernel_at(idx);
@@ -559,6 +614,17 @@ static int32_t gemm_ex(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* desc, const
     if (rc != MAIZE_OK) return rc;
     if (!kernel) {
         const uint32_t cus = (uint32_t)ctx->prop.multiProcessorCount;
+        uint32_t chosen;
+        if ((rc = select_checked(*desc, cus, &chosen)) != MAIZE_OK) return rc;
+        // One of the launcher's own forms, where it is faster (fixed scratch: what the registry's plan does not fit is refused
+        // all the same, as documented).
+        maize::FormPlan form;
+        if (maize::choose_form(*desc, chosen, cus, &form)) {
+            bool ran;
+            if (fixed && (rc = fits_fixed(ctx, desc, chosen, fixed)) != MAIZE_OK) return rc;
+            rc = form_launch(ctx, desc, form, stream, fixed, &ran);
+            if (rc != MAIZE_OK || ran) return rc;
+        }
         // A tile count a little over a whole number of rounds: the leading tile rows (or tile columns) fill the rounds,
         // the rest is a product with few tiles that runs in 128-row tiles or split over K, behind it on the same stream.
         const maize::TailSplit cut = maize::tail_split(*desc, cus);
@@ -593,8 +659,6 @@ static int32_t gemm_ex(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* desc, const
             if (rc != MAIZE_OK) return rc;
             return gemm_launch(ctx, &rest, irest, stream, fixed);
         }
-        uint32_t chosen;
-        if ((rc = select_checked(*desc, cus, &chosen)) != MAIZE_OK) return rc;
         return gemm_launch(ctx, desc, chosen, stream, fixed);
     }
     const int idx = maize::kernel_index(kernel);

@@ -1,0 +1,65 @@
+"""The launcher's own forms without a device: what their code object contains, and the LDS layouts they add."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+import maize_amd as mz
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HSACO = os.path.join(os.path.dirname(mz.LIB_PATH), "maize_forms_gfx950.hsaco")
+OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+
+MAPS = r"""
+#include <cstdio>
+#include <set>
+#include "maps.hpp"
+using namespace maize::maps;
+// a pass (32 lanes, 8 bytes each) of a transposing read hits each of the 64 banks once
+static bool free_of_conflicts(const unsigned (&off)[64]) {
+    for (int p = 0; p < 64; p += 32) {
+        std::set<unsigned> banks;
+        for (int l = p; l < p + 32; ++l) for (unsigned b = 0; b < 8; b += 4) if (!banks.insert((off[l] + b) / 4 % 64).second) return false;
+    }
+    return true;
+}
+int main() {
+    std::set<unsigned> seen, seen8;
+    for (unsigned pc = 0; pc < 8; ++pc) for (unsigned l = 0; l < 64; ++l) {
+        if (sk64_offset(sk64_piece_row(pc, l), sk64_piece_chunk(pc, l)) != pc * 1024 + l * 16 || !seen.insert(sk64_piece_row(pc, l) * 8 + sk64_piece_chunk(pc, l)).second) return 1;
+        if (sk8s_offset(sk8s_piece_row(pc, l), sk8s_piece_chunk(pc, l)) != pc * 1024 + l * 16 || !seen8.insert(sk8s_piece_row(pc, l) * 4 + sk8s_piece_chunk(pc, l)).second) return 2;
+    }
+    for (unsigned cg = 0; cg < 4; ++cg) for (unsigned k = 0; k < 2; ++k) for (unsigned h = 0; h < 2; ++h) {
+        unsigned off[64], off8[64];
+        for (unsigned l = 0; l < 64; ++l) {
+            const unsigned q = l & 15, g = l >> 4;
+            off[l] = sk64_tr_offset(cg, 0, l) + 4096 * k + 512 * h;
+            const unsigned row = 32 * k + 8 * g + 4 * h + q / 4, col = 16 * cg + 4 * (q % 4);
+            if (off[l] != sk64_offset(row, col >> 3) + (col & 7) * 2) return 3;
+            off8[l] = sk8s_tr_offset(cg, 0, 0, l) + 4096 * k + 512 * h;
+            const unsigned row8 = 64 * k + 16 * g + 8 * h + q / 2, col8 = 16 * cg + 8 * (q % 2);
+            if (off8[l] != sk8s_offset(row8, col8 >> 4) + (col8 & 15)) return 4;
+        }
+        if (!free_of_conflicts(off) || !free_of_conflicts(off8)) return 5;
+    }
+    return seen.size() == 64 * 8 && seen8.size() == 128 * 4 ? 0 : 6;
+}
+"""
+
+
+def test_the_64_column_tiles_of_a_row_major_b_are_whole_and_free_of_bank_conflicts(tmp_path):
+    src, exe = tmp_path / "maps.cpp", tmp_path / "maps"
+    src.write_text(MAPS)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "maize_amd", "csrc", "kernels"), "-o", str(exe), str(src)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
+
+
+@pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(HSACO)), reason="needs the ROCm llvm-objdump and the built code object")
+def test_form_kernels_keep_to_registers_and_plain_stores():
+    text = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", HSACO], check=True, capture_output=True, text=True).stdout
+    names = re.findall(r"^[0-9a-f]+ <(maize_[A-Za-z0-9_]+)>:", text, re.M)
+    assert len(names) >= 40
+    for banned in ("scratch_", "v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32", "s_dcache_" + "wb", "s_sto" + "re", "s_ato" + "mic"):
+        assert "\t" + banned not in text, banned

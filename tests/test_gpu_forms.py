@@ -1,0 +1,99 @@
+"""The kernels of the launcher's own forms (maize_amd/csrc/kernels/form_kernels.hip), launched by hand from their code object
+at the sizes where they can go wrong: one element more or less than a tile, a K tile, a 16-byte chunk, a ring of K tiles;
+rows and pointers on no grid; K ranges.  Against the oracle, to the bars of the registry kernels (test_gpu_gemm_ex.py,
+test_gpu_gemm_f8.py)."""
+import os
+
+import numpy as np
+import pytest
+
+import maize_amd as mz
+from maize_amd import _ffi
+
+pytestmark = pytest.mark.gpu
+
+HSACO = os.path.join(os.path.dirname(mz.LIB_PATH), "maize_forms_gfx950.hsaco")
+NN, NT = mz.LAYOUT_NN, mz.LAYOUT_NT
+TILES = {"32x128": (32, 128), "64x64": (64, 64), "64x128": (64, 128), "64x64w": (64, 64)}
+OPS = {"bf16": 0, "f16": 4, "e4m3": 8, "e5m2": 8 | 48, "e4m3e5m2": 8 | 32, "e5m2e4m3": 8 | 16}      # GemmArgs::epi
+
+
+@pytest.fixture(scope="module")
+def forms(ctx):
+    with open(HSACO, "rb") as f:
+        mod = ctx.load_module(f.read())
+    yield mod
+    mod.unload()
+
+
+def operands(oracle, op, count, which, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.random(count) * 2.0 - 1.0
+    if op in ("bf16", "f16"):
+        return oracle.bf16_bits_from_f64(x, oracle.BF16 if op == "bf16" else oracle.F16)
+    fmt = op if len(op) == 4 else op[:4] if which == 0 else op[4:]
+    return oracle.fp8_bits_from_f64(x, {"e4m3": oracle.E4M3, "e5m2": oracle.E5M2}[fmt])
+
+
+def check_form(ctx, oracle, mod, op, tile, layout, m, n, k, ks=1, off=0, pad=0, alpha=1.0, beta=0.0, out_f32=False, batch=1):
+    bm, bn = TILES[tile]
+    name = f"maize_tile_{op}_{'nt' if layout == NT else 'nn'}_{tile}"
+    esz = 2 if op in ("bf16", "f16") else 1
+    brows, bcols = (n, k) if layout == NT else (k, n)
+    lda, ldb, ldc = k + pad, bcols + pad, n + pad
+    sa, sb, sc = m * lda + pad, brows * ldb + pad, m * ldc + pad
+    a, b = operands(oracle, op, batch * sa, 0, 1), operands(oracle, op, batch * sb, 1, 2)
+    c0 = np.random.default_rng(3).random(batch * sc + off).astype(np.float32) if out_f32 else operands(oracle, "f16" if op == "f16" else "bf16", batch * sc + off, 0, 3)
+    place = lambda x: np.concatenate([np.zeros(off, x.dtype), x])
+    da, db, dc = ctx.upload(place(a)), ctx.upload(place(b)), ctx.upload(c0)
+    items = -(-m // bm) * -(-n // bn) * batch * ks
+    ws = ctx.malloc(65536 + items * bm * bn * 4)
+    ws.fill(0)
+    args = _ffi.GemmArgsT(a=da.ptr + off * esz, arows=m, acols=k, b=db.ptr + off * esz, brows=brows, bcols=bcols,
+                          c=dc.ptr + off * c0.itemsize, crows=m, ccols=n, stride_a=sa, stride_b=sb, stride_c=sc, batch=batch, layout=layout,
+                          workspace=ws.ptr, ksplit=ks, lda=lda, ldb=ldb, ldc=ldc,
+                          epi=OPS[op] | (1 if out_f32 else 0) | (2 if (alpha, beta) != (1.0, 0.0) else 0), alpha=alpha, beta=beta)
+    print(f"form {name} {m}x{n}x{k} ks={ks} off={off} pad={pad} batch={batch} f32={out_f32} beta={beta}", flush=True)
+    kern = mod.kernel(name)
+    mz.api.LoadedKernel(ctx, mod, kern, (256, 1, 1)).launch((items, 1, 1), args)
+    ctx.sync()
+    got, left = dc.download(c0.dtype), ws.download(np.uint32, 16384)
+    _ffi.check(_ffi.lib().maize_hip_kernel_release(kern))
+    for x in (da, db, dc, ws):
+        x.free()
+    assert not left.any(), "ticket counters are not back at zero"
+    assert np.array_equal(got[:off], c0[:off])
+    elem = {"bf16": oracle.BF16, "f16": oracle.F16, "e4m3": oracle.E4M3, "e5m2": oracle.E5M2,
+            "e4m3e5m2": (oracle.E4M3, oracle.E5M2), "e5m2e4m3": (oracle.E5M2, oracle.E4M3)}[op]
+    for i in range(batch):
+        gv, ov = got[off + i * sc:][:m * ldc].reshape(m, ldc), c0[off + i * sc:][:m * ldc].reshape(m, ldc)
+        assert np.array_equal(gv[:, n:], ov[:, n:]), "wrote into C's row padding"
+        ref, val, scale = oracle.ref_gemm_ex(a[i * sa:][:m * lda].copy(), b[i * sb:][:brows * ldb].copy(), m, n, k, layout=layout, lda=lda, ldb=ldb, alpha=alpha, beta=beta,
+                                             c_old=None if beta == 0.0 else ov[:, :n].copy(), out_f32=out_f32, elem=elem)
+        f8_unit = esz == 1 and not tile.endswith("w")              # (widened operands: the sums of the 16-bit kernels)
+        if out_f32:
+            tol = ((oracle.floor_coeff_f8(k) + 2.0 ** -23) if f8_unit else (k / 16.0 + 4.0) * 2.0 ** -24) * scale + 1e-45
+            assert (np.abs(gv[:, :n].astype(np.float64) - val) <= tol).all()
+        else:
+            s = oracle.compare(gv[:, :n].copy(), ref, val, scale, k, elem=oracle.F16 if op == "f16" else oracle.BF16,
+                               coeff=oracle.floor_coeff_f8(k) if f8_unit else None)
+            assert s["n_fail"] == 0, s
+            if esz == 2:
+                oracle.assert_parity(s, name)
+
+
+@pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
+@pytest.mark.parametrize("op,tile", [(op, t) for op in OPS for t in TILES if op not in ("bf16", "f16") or t != "64x64w"])
+def test_tile_forms_at_their_edges(ctx, oracle, forms, op, tile, layout):
+    bm, bn = TILES[tile]
+    kt = 64 if op in ("bf16", "f16") else 128
+    ch = kt // 8
+    # K: the shortest, a chunk's and a K tile's edges, whole tiles only, and one entry around a full ring (at most 5 stages)
+    for i, k in enumerate((ch, ch + 1, kt - 1, kt, kt + 1, 3 * kt, 4 * kt + ch, 5 * kt, 5 * kt + 1, 6 * kt + 3, 7 * kt, 8 * kt - 1)):
+        check_form(ctx, oracle, forms, op, tile, layout, bm + (i % 3) - 1, bn + 1 - (i % 3), k, off=i % 2, pad=(0, 3, 8)[i % 3])
+    check_form(ctx, oracle, forms, op, tile, layout, 1, ch, ch)
+    check_form(ctx, oracle, forms, op, tile, layout, 2 * bm + 1, 9 * bn + 3, kt + 9, alpha=-1.25, beta=0.75)     # sweeps of 8 tile rows, ragged
+    check_form(ctx, oracle, forms, op, tile, layout, 8 * bm + 5, 2 * bn - 1, kt, out_f32=True, alpha=0.5, beta=1.0, off=1)
+    check_form(ctx, oracle, forms, op, tile, layout, bm + 1, bn + ch, 2 * kt + 5, batch=3, pad=1)
+    for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)):                                               # K ranges, the tail in the last
+        check_form(ctx, oracle, forms, op, tile, layout, bm + 3, bn + 5, k, ks=ks, out_f32=ks == 3)
