@@ -12,17 +12,22 @@ namespace {
 inline uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 inline uint64_t cdiv64(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
-// ---- maize_tile_*: tiles of 32 x 128, 64 x 64 and 64 x 128 (kernels/gemm_tile.hpp) --------------------------------------
-enum Tile : uint32_t { T32x128, T64x64, T64x128, T64x64W, kTiles };     // W: 8-bit operands widened to bf16
-constexpr const char* const kOperands[6] = {"bf16", "f16", "e4m3", "e5m2", "e4m3e5m2", "e5m2e4m3"};   // maize_in_type_t's order
-constexpr uint32_t kTileForms = 6u * 2u * kTiles;
+// ---- maize_tile_*: tiles of 32 x 128, 64 x 64 and 64 x 128 (kernels/gemm_tile.hpp), fp32 also 128 x 128 -----------------
+enum Tile : uint32_t { T32x128, T64x64, T64x128, T64x64W, T128x128, kTiles };     // W: 8-bit operands widened to bf16
+constexpr const char* const kOperands[8] = {"bf16", "f16", "e4m3", "e5m2", "e4m3e5m2", "e5m2e4m3", "f32", "f64"};   // maize_in_type_t's order
+constexpr uint32_t kTileForms = 8u * 2u * kTiles;
+static_assert(kTileForms <= kMaxForms, "the context's table of functions");
+bool tile_exists(uint32_t in_type, uint32_t tile) {
+    const bool wide = in_type >= MAIZE_IN_F32;
+    return tile == T64x64W ? !wide && in_type >= MAIZE_IN_E4M3 : tile == T128x128 ? in_type == MAIZE_IN_F32 : true;
+}
 struct Names {
     char name[kTileForms][40];
     Names() {
-        static const char* const kShape[kTiles] = {"32x128", "64x64", "64x128", "64x64w"};
+        static const char* const kShape[kTiles] = {"32x128", "64x64", "64x128", "64x64w", "128x128"};
         for (uint32_t i = 0; i < kTileForms; ++i) {
             const uint32_t t = i % kTiles, nt = i / kTiles % 2u, op = i / kTiles / 2u;
-            if (t == T64x64W && op < 2u) name[i][0] = 0;
+            if (!tile_exists(op, t)) name[i][0] = 0;
             else std::snprintf(name[i], sizeof name[i], "maize_tile_%s_%s_%s", kOperands[op], nt ? "nt" : "nn", kShape[t]);
         }
     }
@@ -40,11 +45,23 @@ const Names& names() {
 // rows of A (B) that are no 16-byte material make the requests longer by ua (ub), transposing reads by nn, 8-bit
 // operands by e8; at least bytes / bw.
 struct TileCost { uint32_t bm, bn; double t0, one, many, turn, r0, r1, ua, ub, nn, bw, tail, e8; };
-constexpr TileCost kTileCost[kTiles] = {
+constexpr TileCost kTileCost[T128x128] = {
     {32, 128, 3.62, 0.215, 0.371, 0.0, 1.63, 0.14, 0.18, 0.36, 0.0, 6.55, 0.55, 0.07},
     {64, 64, 3.97, 0.167, 0.177, 1.06, 1.82, 0.19, 0.11, 0.40, 0.14, 6.88, 0.30, 0.10},
     {64, 128, 4.10, 0.278, 0.292, 1.49, 1.33, 0.54, 0.24, 0.25, 0.04, 6.03, 0.29, 0.09},
     {64, 64, 3.57, 0.329, 0.276, 1.27, 2.20, 0.22, 0.12, 0.15, 0.10, 5.21, 0.65, -0.04},
+};
+// fp32 and fp64 operands: bound by the matrix instructions (a K tile of 64 x 64 is 1024 of their cycles, 0.43 us), so alignment
+// and layout cost next to nothing.  Fitted to 18600 timings of 1977 products, residuals 5-6 %.
+constexpr TileCost kFullCost[2][kTiles] = {
+    {{32, 128, 3.48, 0.548, 0.560, 1.82, 2.22, 0.22, 0.0, 0.0, 0.0, 6.49, 0.30, 0.0},
+     {64, 64, 3.50, 0.541, 0.489, 1.90, 2.26, 0.23, 0.0, 0.0, 0.0, 8.34, 0.27, 0.0},
+     {64, 128, 4.12, 1.006, 0.905, 2.83, 1.28, 0.59, 0.0, 0.0, 0.03, 7.19, 0.27, 0.0},
+     {},
+     {128, 128, 4.24, 2.129, 1.876, 3.89, 0.0, 0.0, 0.0, 0.0, 0.0, 4.00, 0.41, 0.0}},
+    {{32, 128, 4.05, 0.532, 0.558, 2.43, 1.71, 0.46, 0.0, 0.0, 0.0, 6.43, 0.29, 0.0},
+     {64, 64, 4.20, 0.524, 0.477, 2.72, 1.55, 0.52, 0.0, 0.0, 0.0, 8.58, 0.11, 0.0},
+     {64, 128, 5.28, 0.968, 0.893, 4.59, 1.42, 1.03, 0.0, 0.0, 0.03, 6.77, 0.17, 0.0}},
 };
 // The longer of two times that overlap, smoothly (their 4-norm).
 inline double longer(double a, double b) {
@@ -128,13 +145,13 @@ const char* form_name(uint32_t index) {
 
 bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t compute_units, FormPlan* out) {
     const Family fam = families()[registry];
-    if (fam == kWide || compute_units == 0u) return false;
+    if (compute_units == 0u) return false;
     Problem p;
     p.s = dims_of(d);
     p.batch = d.gemm.batch;
     p.cus = compute_units;
     const bool bits8 = d.in_type >= MAIZE_IN_E4M3 && d.in_type <= MAIZE_IN_E5M2_E4M3;
-    p.esz = bits8 ? 1u : 2u;
+    p.esz = d.in_type == MAIZE_IN_F64 ? 8u : d.in_type == MAIZE_IN_F32 ? 4u : bits8 ? 1u : 2u;
     p.bke = 128u / p.esz;
     p.steps = cdiv(p.s.k, p.bke);
     p.tail = p.s.k % p.bke != 0u;
@@ -149,13 +166,15 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     };
     p.rows_a = rows16(d.gemm.a.ptr, lda, d.gemm.stride_a);
     p.rows_b = rows16(d.gemm.b.ptr, ldb, d.gemm.stride_b);
-    const double c_bytes = d.out_type == MAIZE_OUT_F32 ? 4.0 : 2.0;
+    const double c_bytes = fam == kWide ? p.esz : d.out_type == MAIZE_OUT_F32 ? 4.0 : 2.0;
     p.bytes = p.batch * (p.esz * ((double)p.s.m + p.s.n) * p.s.k + c_bytes * p.s.m * p.s.n * (d.beta != 0.0f ? 2.0 : 1.0));
 
     LaunchDims ld;
     std::memset(&ld, 0, sizeof ld);
-    double rival = 1e9;
-    if (fam != kAnyShape && kernel_at(registry).plan(d, compute_units, &ld)) rival = registry_cost(fam, p, ld.ksplit);
+    if (!kernel_at(registry).plan(d, compute_units, &ld)) return false;       // (what the registry's kernel refuses stays refused)
+    // fp32 and fp64: the form always.  Of 1977 drawn products the registry's 128 x 128 tiles through registers were ahead of the
+    // best tile on four, by 3 % at most, and 4.3 times as long on average.
+    const double rival = fam == kAnyShape || fam == kWide ? 1e9 : registry_cost(fam, p, ld.ksplit);
 
     // The any-shape kernel multiplies 8-bit operands widened to bf16: its form does too.  Everywhere else the three tiles.
     const bool widened = bits8 && fam == kAnyShape;
@@ -167,13 +186,13 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     const uint32_t ks_lo = pinned && ld.ksplit > 1u ? ld.ksplit : 1u, ks_hi = pinned ? ks_lo : 16u;
     if (pinned && cdiv(cdiv(p.s.k, 32), ks_lo) * 32u != cdiv(p.steps, ks_lo) * 64u && ks_lo > 1u) return false;
     for (uint32_t t = 0; t < kTiles; ++t) {
-        if ((t == T64x64W) != widened) continue;
-        const TileCost& c = kTileCost[t];
+        if ((t == T64x64W) != widened || !tile_exists(d.in_type, t)) continue;
+        const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][t] : kTileCost[t];
         const uint64_t tiles = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch;
         if (tiles > (1u << 24) || (t == T32x128 && p.s.m > 96u)) continue;
         for (uint32_t ks = ks_lo; ks <= ks_hi; ++ks) {
             // K ranges: of three K tiles or more, none empty, two workgroups per compute unit at most
-            if (ks > 1u && (tiles * ks > (pinned ? 8u : 2u) * compute_units || p.steps / ks < 3u)) break;
+            if (ks > 1u && (tiles * ks > (pinned ? 8u : 2u) * compute_units || p.steps / ks < 3u || t == T128x128)) break;
             if (ks > 1u && cdiv(p.steps, cdiv(p.steps, ks)) != ks) continue;
             const double cost = tile_cost(c, p, tiles, ks);
             if (cost < best) { best = cost; tile = t; ranges = ks; }
@@ -182,12 +201,12 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     // The form has to win 10 % by the model: of 590 products the choice is then 1.4 % behind the best of all candidates on
     // average, and six are slower than with the registry kernel alone, by 3 to 19 % (none allowed: 1.86x on average, all: 1.855x).
     if (best >= 0.9 * rival) return false;
-    const TileCost& c = kTileCost[tile];
+    const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][tile] : kTileCost[tile];
     const uint64_t items = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch * ranges;
     out->kernel = (d.in_type * 2u + (p.s.nt ? 1u : 0u)) * kTiles + tile;
     out->grid = (uint32_t)items;
     out->ksplit = ranges;
-    out->workspace_bytes = ranges > 1u ? kTicketBytes + (size_t)items * c.bm * c.bn * 4u : 0u;
+    out->workspace_bytes = ranges > 1u ? kTicketBytes + (size_t)items * c.bm * c.bn * (p.esz == 8u ? 8u : 4u) : 0u;
     return true;
 }
 

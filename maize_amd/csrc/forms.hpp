@@ -12,7 +12,7 @@
 
 namespace maize {
 
-constexpr uint32_t kMaxForms = 64;
+constexpr uint32_t kMaxForms = 80;
 uint32_t form_count();
 const char* form_name(uint32_t index);     // kernel of the tile code object; NULL: an unused index
 

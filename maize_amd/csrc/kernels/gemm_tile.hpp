@@ -25,6 +25,14 @@
 // 1392 22.9 -> 12.8; 32 x 128 for few rows.  Ragged K against copies of the operands in the workspace: 1024 x 3072 x 1999 61.4 -> 25.9,
 // 3 x 4863 x 4281 48.6 -> 12.1, E4M3 19 x 10987 x 1494 50.1 -> 6.8; against the any-shape kernel: 150 x 201 x 333 26.1 -> 5.9, E4M3
 // 128 x 168 x 296 63 -> 5.5.  (Tried and slower: twice the ring depth on one workgroup per compute unit, three stages on three.)
+//
+// fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
+// What bounds them is the matrix pipe: a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
+// A lane's 16-byte chunk feeds four (two) instructions in turn, the same k on both sides, so a K-contiguous operand needs an
+// eighth of the reads of one element per instruction, and the next K tile's reads run behind this one's instructions.  Against
+// 128 x 128 tiles copied through registers, whose reads stand in front of the instructions they feed: 2048^3 fp32 N x K 162.6 ->
+// 129.1 us (0.85 of the pipe), 4096^3 1040 -> 924 (0.95), 4096^3 fp64 2107 -> 1882 (0.93); and where 128-wide tiles leave the
+// chip idle: 1024^3 fp64 149 -> 42, 8 x 7336 x 4464 fp32 and its like 3 to 10 times.
 #pragma once
 #include <type_traits>
 #include "common.hpp"
@@ -57,6 +65,9 @@ template <bool F16> __device__ __forceinline__ void mfma16(floatx4& c, u32x4 b, 
     if constexpr (F16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
     else               asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a));
 }
+// One element of a row-major 4- or 8-byte B.
+template <int OFF> __device__ __forceinline__ void rd_elem(uint32_t& dst, uint32_t base) { asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "n"(OFF)); }
+template <int OFF> __device__ __forceinline__ void rd_elem(u32x2& dst, uint32_t base) { asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "n"(OFF)); }
 // (B first, so cbsz carries B's format and blgp A's: 0 = E4M3, 1 = E5M2)
 template <int A_E5M2, int B_E5M2> __device__ __forceinline__ void mfma8(floatx4& c, u32x4 b0, u32x4 b1, u32x4 a0, u32x4 a1) {
     typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -88,21 +99,26 @@ __device__ __forceinline__ void drain(uint32_t s, uint32_t ns, F&& f) {
     }
 }
 
-// The layout of a row-major (K x N) B tile BN columns wide (maps.hpp): 64 rows of 16-bit or 128 rows of 8-bit elements.
-template <bool IS8, int BN>
+// The layout of a row-major (K x N) B tile BN columns wide (maps.hpp): 128 / ES rows of elements of ES bytes.
+template <uint32_t ES, int BN>
 struct KN {
+    static constexpr bool IS8 = ES == 1u;
+    static constexpr uint32_t RB = BN * ES;                           // bytes per row
     static constexpr int HALF = BN * (IS8 ? 8 : 8);                   // register half h: 8 rows of 8-bit, 4 rows of 16-bit elements
     static constexpr int DEEP = BN * 64;                              // K half: 64 rows of 8-bit, 32 rows of 16-bit elements
     static __device__ __forceinline__ uint32_t row(uint32_t piece, uint32_t lane) {
-        if constexpr (IS8) return BN == 128 ? maps::sk8n_piece_row(piece, lane) : maps::sk8s_piece_row(piece, lane);
+        if constexpr (ES >= 4u) return maps::we_piece_row(RB, piece, lane);
+        else if constexpr (IS8) return BN == 128 ? maps::sk8n_piece_row(piece, lane) : maps::sk8s_piece_row(piece, lane);
         else               return BN == 128 ? maps::sk128_piece_row(piece, lane) : maps::sk64_piece_row(piece, lane);
     }
     static __device__ __forceinline__ uint32_t chunk(uint32_t piece, uint32_t lane) {
-        if constexpr (IS8) return BN == 128 ? maps::sk8n_piece_chunk(piece, lane) : maps::sk8s_piece_chunk(piece, lane);
+        if constexpr (ES >= 4u) return maps::we_piece_chunk(ES, RB, piece, lane);
+        else if constexpr (IS8) return BN == 128 ? maps::sk8n_piece_chunk(piece, lane) : maps::sk8s_piece_chunk(piece, lane);
         else               return BN == 128 ? maps::sk128_piece_chunk(piece, lane) : maps::sk64_piece_chunk(piece, lane);
     }
     static __device__ __forceinline__ uint32_t read(uint32_t cg, uint32_t lane) {
-        if constexpr (IS8) return BN == 128 ? maps::sk8n_tr_offset(cg, 0, 0, lane) : maps::sk8s_tr_offset(cg, 0, 0, lane);
+        if constexpr (ES >= 4u) return maps::we_read(ES, RB, cg, lane);
+        else if constexpr (IS8) return BN == 128 ? maps::sk8n_tr_offset(cg, 0, 0, lane) : maps::sk8s_tr_offset(cg, 0, 0, lane);
         else               return BN == 128 ? maps::sk128_tr_offset(cg, 0, lane) : maps::sk64_tr_offset(cg, 0, lane);
     }
 };
@@ -152,6 +168,38 @@ __device__ __forceinline__ void store_c8(const GemmArgs& p, void* c, uint64_t at
     }
 }
 
+// fp32 and fp64 C: the 16 bytes of a row of C from element `at` on (the first `count` elements), C = alpha * A.B + beta * C in
+// the operands' type.
+template <class T>
+__device__ __forceinline__ void store_c16(const GemmArgs& p, T* c, uint64_t at, u32x4 v, uint32_t count) {
+    constexpr uint32_t CH = 16u / sizeof(T);
+    const T alpha = (T)p.alpha, beta = (T)p.beta;
+    const bool whole = count >= CH;
+    T x[CH], old[CH];
+    __builtin_memcpy(x, &v, 16);
+    if (p.epi & EPI_SCALE) {
+#pragma unroll
+        for (uint32_t e = 0; e < CH; ++e) old[e] = (T)0;
+        if (beta != (T)0) {
+            if (whole) __builtin_memcpy(old, c + at, 16);
+            else {
+#pragma unroll
+                for (uint32_t e = 0; e < CH; ++e) if (e < count) old[e] = c[at + e];
+            }
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < CH; ++e) {
+            if constexpr (sizeof(T) == 4) x[e] = __builtin_fmaf(beta, old[e], alpha * x[e]);
+            else                          x[e] = __builtin_fma(beta, old[e], alpha * x[e]);
+        }
+    }
+    if (whole) __builtin_memcpy(c + at, x, 16);
+    else {
+#pragma unroll
+        for (uint32_t e = 0; e < CH; ++e) if (e < count) c[at + e] = x[e];
+    }
+}
+
 // Eight E4M3 (E5M2) values as bf16 (exact: bf16 holds every value of both formats).
 template <int E5M2>
 __device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
@@ -166,21 +214,24 @@ __device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
     return bf16x8{w[0][0], w[0][1], w[1][0], w[1][1], w[2][0], w[2][1], w[3][0], w[3][1]};
 }
 
-// ET: 0 bf16, 1 IEEE half, 2 + (A is E5M2) + 2 (B is E5M2): 8-bit operands.
+// ET: 0 bf16, 1 IEEE half, 2 + (A is E5M2) + 2 (B is E5M2): 8-bit operands, 6 fp32, 7 fp64.
 // WIDE: 8-bit operands widened to bf16 as their fragments are read (exact) and multiplied by the bf16 instruction: the
 // arithmetic of the any-shape kernel, which small 8-bit products get.
 // 4 waves as WM x WN, each MI x NJ accumulators of 16 x 16; NS ring stages.
 template <int ET, bool WIDE, bool NT, int BM, int BN, int NS>
 __device__ __forceinline__ void body(const GemmArgs& p) {
-    constexpr bool IS8 = ET >= 2, F16 = ET == 1, TR8 = IS8 && !NT;
+    constexpr bool IS8 = ET >= 2 && ET < 6, F16 = ET == 1, FP = ET >= 6;
     static_assert(!WIDE || IS8, "only 8-bit operands are widened");
-    constexpr uint32_t ES = IS8 ? 1u : 2u, CH = 16u / ES, BKE = 128u / ES;
+    constexpr uint32_t ES = IS8 ? 1u : ET == 6 ? 4u : ET == 7 ? 8u : 2u, CH = 16u / ES, BKE = 128u / ES;
+    constexpr uint32_t AS = ET == 7 ? 8u : 4u;                        // bytes of an accumulator
+    typedef std::conditional_t<ET == 7, double, float> acc_t;
+    typedef acc_t accx4 __attribute__((ext_vector_type(4)));
     constexpr int WN = BM == 32 ? 4 : 2, WM = 4 / WN;
     constexpr int MI = BM / WM / 16, NJ = BN / WN / 16, NMF = MI * NJ;
     constexpr int PA = BM / 32, PB = BN / 32, P = PA + PB;            // 1 KiB requests per wave and K tile
     constexpr uint32_t ASTAGE = BM * 128u, BSTAGE = BN * 128u;
-    typedef KN<IS8, BN> KNB;
-    static_assert(NS * (BM + BN) * 128 >= BM * BN * 4, "the epilogue's fp32 tile takes the ring's place");
+    typedef KN<ES, BN> KNB;
+    static_assert(NS * (BM + BN) * 128u >= BM * BN * AS, "the epilogue's fp32 tile takes the ring's place");
     __shared__ __attribute__((aligned(1024))) char lds_a[NS * (ASTAGE + BSTAGE)];
     char* const lds_b = lds_a + NS * ASTAGE;
     typedef __attribute__((address_space(3))) void* lvp;
@@ -268,15 +319,17 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
         for (int q = 0; q < P; ++q) piece(r, q);
     };
 
-    floatx4 acc[MI][NJ];
+    accx4 acc[MI][NJ];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NJ; ++j) acc[i][j] = accx4{0, 0, 0, 0};
 
     // ---- the tail's loads, then the ring's first NS entries ----------------------------------------------------------
+    // (128 x 128: when they are placed, there are no registers to hold them through the loop)
+    constexpr bool LATE_TAIL = BM * BN > 64 * 128;
     u32x4 ta[PA], tb[PB];
-    if (tail_here) {
+    auto load_tail = [&] {
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
             const uint32_t pc = wave * PA + i, k = k_main + maps::kc_piece_chunk(pc, lane) * CH, row = m0 + maps::kc_piece_row(pc, lane);
@@ -293,10 +346,12 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
                 tb[i] = load16(Bb + ((uint64_t)(k < K ? k : K - 1u) * ldb + (col < N - CH ? col : N - CH)) * ES);
             }
         }
-    }
+    };
+    if (tail_here && !LATE_TAIL) load_tail();
     // ... into ring stage st: a chunk that would have run past the end was loaded from further in front and moves down; K past
     // the end is zero.
     auto place_tail = [&](uint32_t st) {
+        if constexpr (LATE_TAIL) load_tail();
         auto put = [&](uint32_t at, u32x4 v, uint32_t want, uint32_t last, bool live) {
             asm volatile("ds_write_b128 %0, %1" :: "v"(at), "v"(drop_low(v, live ? (want > last ? want - last : 0u) * ES : 16u)) : "memory");
         };
@@ -325,12 +380,13 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
 
     // Fragment reads (maps.hpp): one base per K half (K-contiguous tiles; fragment f sits 2048 f bytes further on) or per
     // column group (K x N tile).
+    const uint32_t b_lane = FP ? (lane & 48u) | maps::we_column(ES, lane) : lane;      // fp64: the fragment's columns in the order of the results
     uint32_t a_rd[2], b_rd[NT ? 2 : NJ];
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) a_rd[kh] = (uint32_t)(uintptr_t)(lds_ptr)lds_a + maps::kc_frag16_offset(wm * (MI * 16u), kh, lane);
     if constexpr (NT) {
 #pragma unroll
-        for (int kh = 0; kh < 2; ++kh) b_rd[kh] = (uint32_t)(uintptr_t)(lds_ptr)lds_b + maps::kc_frag16_offset(wn * (NJ * 16u), kh, lane);
+        for (int kh = 0; kh < 2; ++kh) b_rd[kh] = (uint32_t)(uintptr_t)(lds_ptr)lds_b + maps::kc_frag16_offset(wn * (NJ * 16u), kh, b_lane);
     } else {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) b_rd[j] = (uint32_t)(uintptr_t)(lds_ptr)lds_b + KNB::read(wn * NJ + j, lane);
@@ -341,16 +397,23 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     // behind the MFMAs.  One LDS round trip per step, with one wave per SIMD to hide it: reading K half by K half -- two round
     // trips -- 256 x 256 x 4096 on 16 workgroups took 17.6 us against 16.7 (and 14.4 with no requests past the end).
     // (The waits name every register the reads fill, so that nothing derived from them can move in front.)
-    constexpr int NR = MI * 2 + NJ * (NT ? 2 : 4);                    // reads of a K tile
-    constexpr int NM = IS8 ? NMF : 2 * NMF;                           // its matrix instructions
+    // 4- and 8-byte operands: a lane's 16-byte chunk (row-major B: its CH rows of one column) feeds CH instructions four deep,
+    // the same k on both sides.
+    constexpr int BR = ET == 6 ? 8 : 4;                               // reads of a fragment of a row-major B
+    constexpr int NR = MI * 2 + NJ * (NT ? 2 : BR);                   // reads of a K tile
+    constexpr int NM = FP ? 2 * (int)CH * NMF : IS8 ? NMF : 2 * NMF;  // its matrix instructions
+    typedef std::conditional_t<ET == 6, uint32_t, u32x2> tr_t;
     constexpr int RPS = (NR + NM - 1) / NM;
     u32x4 fa[2][MI][2], fb[2][NT ? NJ : 1][2];                        // set, fragment, K half (8-bit: the lane's chunks l / 16 and 4 + l / 16)
-    u32x2 ft[2][NT ? 1 : NJ][4];                                      // row-major B: set, fragment, 2 (K half) + register half
+    tr_t ft[2][NT ? 1 : NJ][BR];                                      // row-major B: set, fragment, 2 (K half) + register half, or CH (K half) + row
     auto read_one = [&](auto set, auto q_, uint32_t ao, uint32_t bo) {
         constexpr int S = decltype(set)::value, q = decltype(q_)::value;
         if constexpr (q < 2 * MI) rd128<(q % MI) * 2048>(fa[S][q % MI][q / MI], a_rd[q / MI] + ao);
         else if constexpr (NT) rd128<((q - 2 * MI) % NJ) * 2048>(fb[S][(q - 2 * MI) % NJ][(q - 2 * MI) / NJ], b_rd[(q - 2 * MI) / NJ] + bo);
-        else {
+        else if constexpr (FP) {
+            constexpr int r = q - 2 * MI, f = r % NJ, k = r / NJ;     // K half k / CH, element k % CH
+            rd_elem<(k / (int)CH * (int)(BKE / 2u) + k % (int)CH) * (int)KNB::RB>(ft[S][f][k], b_rd[f] + bo);
+        } else {
             constexpr int r = q - 2 * MI, f = (r >> 1) % NJ, kh = (r >> 1) / NJ, h = r & 1;
             rd_tr<IS8, kh * KNB::DEEP + h * KNB::HALF>(ft[S][f][2 * kh + h], b_rd[f] + bo);
         }
@@ -363,18 +426,37 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             if constexpr (NT) pin(fb[S][j][0], fb[S][j][1]);
-            else { pin(ft[S][j][0], ft[S][j][1]); pin(ft[S][j][2], ft[S][j][3]); }
+            else {
+#pragma unroll
+                for (int e = 0; e < BR; e += 2) pin(ft[S][j][e], ft[S][j][e + 1]);
+            }
         }
     };
     auto b_half = [&](auto set, int j, int kh) -> u32x4 {
         constexpr int S = decltype(set)::value;
         if constexpr (NT) return fb[S][j][kh];
+        else if constexpr (FP) return u32x4{0u, 0u, 0u, 0u};
         else return u32x4{ft[S][j][2 * kh][0], ft[S][j][2 * kh][1], ft[S][j][2 * kh + 1][0], ft[S][j][2 * kh + 1][1]};
     };
     // Matrix instruction n of a K tile (B's fragment first: a lane ends up with 4 consecutive columns of one row of C).
     auto multiply = [&](auto set, auto n_) {
         constexpr int S = decltype(set)::value, n = decltype(n_)::value, i = n % NMF / NJ, j = n % NJ;
-        if constexpr (!IS8) mfma16<F16>(acc[i][j], b_half(set, j, n / NMF), fa[S][i][n / NMF]);
+        if constexpr (FP) {
+            // (the compiler's own instruction: it knows these, slower, pipelines' hazards)
+            constexpr int k = n / NMF, kh = k / (int)CH, e = k % (int)CH;
+            const u32x4 a = fa[S][i][kh];
+            if constexpr (ET == 6) {
+                const uint32_t av = a[e];                             // (a bit cast of the vector's element itself takes element 0)
+                uint32_t bv;
+                if constexpr (NT) bv = fb[S][j][kh][e]; else bv = ft[S][j][k];
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, bv), __builtin_bit_cast(float, av), acc[i][j], 0, 0, 0);
+            } else {
+                u32x2 b;
+                if constexpr (NT) b = u32x2{fb[S][j][kh][2 * e], fb[S][j][kh][2 * e + 1]}; else b = ft[S][j][k];
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(__builtin_bit_cast(double, b), __builtin_bit_cast(double, u32x2{a[2 * e], a[2 * e + 1]}), acc[i][j], 0, 0, 0);
+            }
+        }
+        else if constexpr (!IS8) mfma16<F16>(acc[i][j], b_half(set, j, n / NMF), fa[S][i][n / NMF]);
         else if constexpr (!WIDE) mfma8<(ET - 2) & 1, ((ET - 2) >> 1)>(acc[i][j], b_half(set, j, 0), b_half(set, j, 1), fa[S][i][0], fa[S][i][1]);
     };
     uint32_t st = 0u;                                                 // ring stage of the entry in hand
@@ -443,14 +525,19 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     // ---- K ranges: the last to arrive adds the partial tiles in range order -----------------------------------
     if (ks > 1u) {
         constexpr int COHERENT = 17;                                  // sc0 | sc1: these accesses cross the per-XCD L2s
-        constexpr uint32_t PART = BM * BN * 4u;
-        constexpr int ZG = NMF <= 4 ? 8 : 2;                          // ranges whose loads are in flight at a time
+        constexpr uint32_t PART = BM * BN * AS;
+        constexpr int AW = AS / 4;                                    // 16-byte words of an accumulator
+        constexpr int ZG = (NMF <= 4 ? 8 : 2) / AW;                   // ranges whose loads are in flight at a time
+        struct Words { u32x4 w[AW]; };
         uint32_t* const counters = (uint32_t*)p.workspace;            // zero between launches
         const __amdgpu_buffer_rsrc_t rws = make_rsrc((const char*)p.workspace + 65536, total * PART);
         const uint32_t mine = item * PART + tid * 16u, first = t * ks * PART + tid * 16u;
 #pragma unroll
-        for (int q = 0; q < NMF; ++q)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[q / NJ][q % NJ]), rws, mine + q * 4096u, 0, COHERENT);
+        for (int q = 0; q < NMF; ++q) {
+            const Words x = __builtin_bit_cast(Words, acc[q / NJ][q % NJ]);
+#pragma unroll
+            for (int h = 0; h < AW; ++h) __builtin_amdgcn_raw_buffer_store_b128(x.w[h], rws, mine + (q * AW + h) * 4096u, 0, COHERENT);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // this wave's part has reached memory
         volatile uint32_t* const ticket = (volatile uint32_t*)lds_a;   // (the ring is idle: a word of its own would cost the second workgroup of the compute unit)
         __syncthreads();
@@ -458,12 +545,17 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
         __syncthreads();
         if (*ticket != ks - 1u) return;
         for (uint32_t z0 = 0; z0 < ks; z0 += ZG) {
-            floatx4 part[ZG][NMF];
+            accx4 part[ZG][NMF];
 #pragma unroll
             for (int u = 0; u < ZG; ++u)
 #pragma unroll
-                for (int q = 0; q < NMF; ++q)
-                    part[u][q] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rws, z0 + u < ks ? first + (z0 + u) * PART + q * 4096u : 0xFFFFFFF0u, 0, COHERENT));
+                for (int q = 0; q < NMF; ++q) {
+                    Words x;
+#pragma unroll
+                    for (int h = 0; h < AW; ++h)
+                        x.w[h] = __builtin_amdgcn_raw_buffer_load_b128(rws, z0 + u < ks ? first + (z0 + u) * PART + (q * AW + h) * 4096u : 0xFFFFFFF0u, 0, COHERENT);
+                    part[u][q] = __builtin_bit_cast(accx4, x);
+                }
 #pragma unroll
             for (int u = 0; u < ZG; ++u)
 #pragma unroll
@@ -483,17 +575,33 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     // code once, and fetching it is what a long one costs.
     lds_ptr const ew = (lds_ptr)lds_a;
     __syncthreads();                                                  // (every wave's requests have landed, the ticket has been read)
+    // (an fp64 accumulator is two chunks)
+    constexpr uint32_t CW = AS / 4u;
     {
         const uint32_t l16 = lane & 15u, g = lane >> 4;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                const uint32_t row = (wm * MI + i) * 16u + l16, chunk = (wn * NJ + j) * 4u + g;
-                *(__attribute__((address_space(3))) floatx4*)(ew + row * (BN * 4u) + ((chunk ^ l16) * 16u)) = acc[i][j];
+                const uint32_t row = (wm * MI + i) * 16u + l16, chunk = ((wn * NJ + j) * 4u + g) * CW;
+                struct Words { u32x4 w[CW]; };
+                const Words x = __builtin_bit_cast(Words, acc[i][j]);
+#pragma unroll
+                for (uint32_t h = 0; h < CW; ++h)
+                    *(__attribute__((address_space(3))) u32x4*)(ew + row * (BN * AS) + (((chunk + h) ^ l16) * 16u)) = x.w[h];
             }
     }
     __syncthreads();
+    if constexpr (FP) {
+        acc_t* const Ct = (acc_t*)p.c + (uint64_t)bz * p.stride_c;
+#pragma unroll 1
+        for (uint32_t r = tid; r < BM * BN / CH; r += 256u) {
+            const uint32_t row = r / (BN / CH), c = r % (BN / CH), grow = m0 + row, gcol = n0 + c * CH;
+            if (grow >= M || gcol >= N) continue;
+            store_c16<acc_t>(p, Ct, (uint64_t)grow * ldc + gcol, *(__attribute__((address_space(3))) u32x4*)(ew + row * (BN * AS) + (c ^ (row & 15u)) * 16u), N - gcol);
+        }
+        return;
+    }
     void* const Cg = (char*)p.c + (uint64_t)bz * p.stride_c * ((p.epi & EPI_F32) ? 4u : 2u);
 #pragma unroll 1
     for (uint32_t r = tid; r < BM * BN / 8u; r += 256u) {
@@ -532,8 +640,20 @@ MAIZE_TILE_8(e4m3, 2)
 MAIZE_TILE_8(e5m2, 5)
 MAIZE_TILE_8(e4m3e5m2, 4)
 MAIZE_TILE_8(e5m2e4m3, 3)
+#define MAIZE_TILE_FP(tag, et) \
+    MAIZE_TILE(maize_tile_##tag##_nn_64x64, et, false, false, 64, 64, 5, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nt_64x64, et, false, true, 64, 64, 5, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nn_32x128, et, false, false, 32, 128, 4, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2)
+MAIZE_TILE_FP(f32, 6)
+MAIZE_TILE_FP(f64, 7)
+MAIZE_TILE(maize_tile_f32_nn_128x128, 6, false, false, 128, 128, 2, 2)
+MAIZE_TILE(maize_tile_f32_nt_128x128, 6, false, true, 128, 128, 2, 2)
 #undef MAIZE_TILE_16
 #undef MAIZE_TILE_8
+#undef MAIZE_TILE_FP
 #undef MAIZE_TILE
 
 }  // namespace maize

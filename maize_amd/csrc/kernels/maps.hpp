@@ -172,5 +172,26 @@ MAIZE_MAP uint32_t sk8s_tr_offset(uint32_t cg, uint32_t kk, uint32_t h, uint32_t
     return sk8s_offset(sk8_tr_row(kk, h, lane), cg) + (lane & 1u) * 8u;
 }
 
+// ---- K x N operand tile of 4-byte (32 rows) or 8-byte elements (16 rows), 64 or 128 columns: no transposing read --------
+// `rb` bytes per row; lane l of piece p lands at byte 1024 p + 16 l.  One-element reads for MFMA 16x16x4: lane group g = l/16
+// needs rows 16 kh + 4 g + e (4-byte, e = 0..3; a pass is all 64 lanes) or 8 kh + 2 g + e (8-byte, e = 0, 1; a pass is 32 lanes)
+// of 16 neighbouring columns (4 or 8 chunks), so the chunk index is XOR-ed with 4 (row/4 % 4) or 8 (row/2 % 2), which moves the
+// groups of a pass to banks of their own.  kh and e stay out of the swizzle: whole rows behind one address register.
+MAIZE_MAP uint32_t we_swizzle(uint32_t es, uint32_t row) { return es == 4u ? 4u * ((row >> 2) & 3u) : 8u * ((row >> 1) & 1u); }
+MAIZE_MAP uint32_t we_piece_row(uint32_t rb, uint32_t piece, uint32_t lane) { return (piece * 1024u + lane * 16u) / rb; }
+MAIZE_MAP uint32_t we_piece_chunk(uint32_t es, uint32_t rb, uint32_t piece, uint32_t lane) {
+    return ((piece * 1024u + lane * 16u) % rb) / 16u ^ we_swizzle(es, we_piece_row(rb, piece, lane));
+}
+MAIZE_MAP uint32_t we_offset(uint32_t es, uint32_t rb, uint32_t row, uint32_t col) {
+    return row * rb + ((col * es / 16u ^ we_swizzle(es, row)) * 16u) + col * es % 16u;
+}
+// The column of a 16-wide fragment that lane l feeds as the first operand, so that its four results are columns
+// 4 (l/16) + 0..3: in order for the fp32 instruction (results are rows 4 (l/16) + v), 0, 4, 8, 12, 1, 5, ... for the fp64 one
+// (rows 4 v + l/16).
+MAIZE_MAP uint32_t we_column(uint32_t es, uint32_t lane) { return es == 4u ? lane & 15u : 4u * (lane & 3u) + ((lane >> 2) & 3u); }
+MAIZE_MAP uint32_t we_read(uint32_t es, uint32_t rb, uint32_t cg, uint32_t lane) {
+    return we_offset(es, rb, (es == 4u ? 4u : 2u) * (lane >> 4), cg * 16u + we_column(es, lane));
+}
+
 }  // namespace maps
 }  // namespace maize

@@ -44,6 +44,27 @@ int main() {
         }
         if (!free_of_conflicts(off) || !free_of_conflicts(off8)) return 5;
     }
+    // 4- and 8-byte elements, 64 and 128 columns: every chunk once, and the reads of a pass (64 or 32 lanes) on banks of their own
+    for (unsigned es : {4u, 8u}) for (unsigned bn : {64u, 128u}) {
+        const unsigned rb = es * bn, rows = 128 / es, ch = 16 / es;
+        std::set<unsigned> all;
+        for (unsigned pc = 0; pc < bn / 8; ++pc) for (unsigned l = 0; l < 64; ++l) {
+            const unsigned row = we_piece_row(rb, pc, l), chunk = we_piece_chunk(es, rb, pc, l);
+            if (we_offset(es, rb, row, chunk * ch) != pc * 1024 + l * 16 || row >= rows || chunk * 16 >= rb || !all.insert(row * 256 + chunk).second) return 7;
+        }
+        if (all.size() != bn * 8) return 8;
+        for (unsigned cg = 0; cg < bn / 16; ++cg) for (unsigned kh = 0; kh < 2; ++kh) for (unsigned e = 0; e < ch; ++e) {
+            std::set<unsigned> banks, cols;
+            for (unsigned l = 0; l < 64; ++l) {
+                if (es == 8 && l % 32 == 0) banks.clear();
+                const unsigned off = we_read(es, rb, cg, l) + (kh * rows / 2 + e) * rb;
+                if (off != we_offset(es, rb, kh * rows / 2 + ch * (l >> 4) + e, 16 * cg + we_column(es, l))) return 9;
+                for (unsigned b = 0; b < es; b += 4) if (!banks.insert((off + b) / 4 % 64).second) return 10;
+                cols.insert(we_column(es, l));
+            }
+            if (cols.size() != 16) return 11;
+        }
+    }
     return seen.size() == 64 * 8 && seen8.size() == 128 * 4 ? 0 : 6;
 }
 """

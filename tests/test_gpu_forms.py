@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 HSACO = os.path.join(os.path.dirname(mz.LIB_PATH), "maize_forms_gfx950.hsaco")
 NN, NT = mz.LAYOUT_NN, mz.LAYOUT_NT
-TILES = {"32x128": (32, 128), "64x64": (64, 64), "64x128": (64, 128), "64x64w": (64, 64)}
+TILES = {"32x128": (32, 128), "64x64": (64, 64), "64x128": (64, 128), "64x64w": (64, 64), "128x128": (128, 128)}
 OPS = {"bf16": 0, "f16": 4, "e4m3": 8, "e5m2": 8 | 48, "e4m3e5m2": 8 | 32, "e5m2e4m3": 8 | 16}      # GemmArgs::epi
 
 
@@ -83,7 +83,7 @@ def check_form(ctx, oracle, mod, op, tile, layout, m, n, k, ks=1, off=0, pad=0, 
 
 
 @pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
-@pytest.mark.parametrize("op,tile", [(op, t) for op in OPS for t in TILES if op not in ("bf16", "f16") or t != "64x64w"])
+@pytest.mark.parametrize("op,tile", [(op, t) for op in OPS for t in TILES if t != "128x128" and (op not in ("bf16", "f16") or t != "64x64w")])
 def test_tile_forms_at_their_edges(ctx, oracle, forms, op, tile, layout):
     bm, bn = TILES[tile]
     kt = 64 if op in ("bf16", "f16") else 128
@@ -97,3 +97,51 @@ def test_tile_forms_at_their_edges(ctx, oracle, forms, op, tile, layout):
     check_form(ctx, oracle, forms, op, tile, layout, bm + 1, bn + ch, 2 * kt + 5, batch=3, pad=1)
     for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)):                                               # K ranges, the tail in the last
         check_form(ctx, oracle, forms, op, tile, layout, bm + 3, bn + 5, k, ks=ks, out_f32=ks == 3)
+
+
+@pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
+@pytest.mark.parametrize("ty,tile", [(ty, t) for ty in ("f32", "f64") for t in ("32x128", "64x64", "64x128", "128x128") if (ty, t) != ("f64", "128x128")])
+def test_full_precision_forms_at_their_edges(ctx, oracle, forms, ty, tile, layout):
+    bm, bn = TILES[tile]
+    dt, kt = (np.float32, 32) if ty == "f32" else (np.float64, 16)
+    es, ch = np.dtype(dt).itemsize, 16 // np.dtype(dt).itemsize
+
+    def check(m, n, k, ks=1, off=0, pad=0, alpha=1.0, beta=0.0, batch=1):
+        name = f"maize_tile_{ty}_{'nt' if layout == NT else 'nn'}_{tile}"
+        print(f"form {name} {m}x{n}x{k} ks={ks} off={off} pad={pad} batch={batch} beta={beta}", flush=True)
+        brows, bcols = (n, k) if layout == NT else (k, n)
+        lda, ldb, ldc = k + pad, bcols + pad, n + pad
+        sa, sb, sc = m * lda + pad, brows * ldb + pad, m * ldc + pad
+        rng = np.random.default_rng(7)
+        a, b, c0 = ((rng.random(off + batch * x) * 2 - 1).astype(dt) for x in (sa, sb, sc))
+        da, db, dc = ctx.upload(a), ctx.upload(b), ctx.upload(c0)
+        items = -(-m // bm) * -(-n // bn) * batch * ks
+        ws = ctx.malloc(65536 + items * bm * bn * es)
+        ws.fill(0)
+        args = _ffi.GemmArgsT(a=da.ptr + off * es, arows=m, acols=k, b=db.ptr + off * es, brows=brows, bcols=bcols, c=dc.ptr + off * es,
+                              crows=m, ccols=n, stride_a=sa, stride_b=sb, stride_c=sc, batch=batch, layout=layout, workspace=ws.ptr, ksplit=ks,
+                              lda=lda, ldb=ldb, ldc=ldc, epi=2 if (alpha, beta) != (1.0, 0.0) else 0, alpha=alpha, beta=beta)
+        kern = forms.kernel(name)
+        mz.api.LoadedKernel(ctx, forms, kern, (256, 1, 1)).launch((items, 1, 1), args)
+        ctx.sync()
+        got, left = dc.download(dt), ws.download(np.uint32, 16384)
+        _ffi.check(_ffi.lib().maize_hip_kernel_release(kern))
+        for x in (da, db, dc, ws):
+            x.free()
+        assert not left.any(), "ticket counters are not back at zero"
+        for i in range(batch):
+            cut = lambda x, s, r, ld: x[off + i * s:][:r * ld].reshape(r, ld)
+            gv, ov = cut(got, sc, m, ldc), cut(c0, sc, m, ldc)
+            assert np.array_equal(gv[:, n:], ov[:, n:]), "wrote into C's row padding"
+            hi, lo, ab = oracle.ref_gemm_wide(np.ascontiguousarray(cut(a, sa, m, lda)[:, :k]), np.ascontiguousarray(cut(b, sb, brows, ldb)[:, :bcols]), m, n, k, layout=layout)
+            worst = oracle.check_wide(gv[:, :n], hi.reshape(m, n), lo.reshape(m, n), ab.reshape(m, n), k, alpha, beta, ov[:, :n])
+            assert worst <= 1.0, worst
+
+    # K: the shortest, a chunk's and a K tile's edges, whole tiles only, and one entry around a full ring (at most 5 stages)
+    for i, k in enumerate((ch, ch + 1, kt - 1, kt, kt + 1, 3 * kt, 4 * kt + ch, 5 * kt, 5 * kt + 1, 6 * kt + 3, 7 * kt, 8 * kt - 1)):
+        check(bm + (i % 3) - 1, bn + 1 - (i % 3), k, off=i % 2, pad=(0, 3, 8)[i % 3])
+    check(1, ch, ch)
+    check(2 * bm + 1, 9 * bn + 3, kt + 9, alpha=-1.25, beta=0.75)
+    check(bm + 1, bn + ch, 2 * kt + 5, batch=3, pad=1)
+    for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)) if tile != "128x128" else ():      # (never split)
+        check(bm + 3, bn + 5, k, ks=ks)
