@@ -569,8 +569,9 @@ static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint
                       sizeof args);
 }
 
-// Runs one of the launcher's own forms.  *ran = false: it cannot be run here (its workspace would have to be allocated while
-// the stream is being captured, which the registry kernel may not need): nothing was launched.
+// Runs one of the launcher's own forms.  *ran = false: it cannot be run here, nothing was launched.  A form with K ranges
+// stays out of captured graphs: a graph keeps the address of the stream's workspace, which a later, larger product frees,
+// and the registry kernel may need none.
 static int32_t form_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, const maize::FormPlan& f, void* stream,
                            const maize_workspace* fixed, bool* ran) {
     maize_gemm_args_t args = args_of(x);
@@ -580,10 +581,12 @@ static int32_t form_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, cons
         if (f.workspace_bytes > fixed->bytes) return MAIZE_OK;
         args.workspace = fixed->ptr;
     } else if (f.workspace_bytes) {
-        if (ctx->workspaces[stream].bytes < f.workspace_bytes) {
-            hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-            if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return MAIZE_OK;
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) {
+            (void)hipGetLastError();                                  // (the null stream, while another one is captured)
+            return MAIZE_OK;
         }
+        if (capturing != hipStreamCaptureStatusNone) return MAIZE_OK;
         int32_t rc = workspace_for(ctx, stream, f.workspace_bytes, &args.workspace);
         if (rc != MAIZE_OK) return rc;
     }

@@ -2,6 +2,7 @@
 at the sizes where they can go wrong: one element more or less than a tile, a K tile, a 16-byte chunk, a ring of K tiles;
 rows and pointers on no grid; K ranges.  Against the oracle, to the bars of the registry kernels (test_gpu_gemm_ex.py,
 test_gpu_gemm_f8.py)."""
+import ctypes as C
 import os
 
 import numpy as np
@@ -145,3 +146,44 @@ def test_full_precision_forms_at_their_edges(ctx, oracle, forms, ty, tile, layou
     check(bm + 1, bn + ch, 2 * kt + 5, batch=3, pad=1)
     for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)) if tile != "128x128" else ():      # (never split)
         check(bm + 3, bn + 5, k, ks=ks)
+
+
+def test_captured_products_keep_no_address_of_a_workspace_that_may_be_freed(ctx):
+    """A product whose form splits K, captured where the stream's workspace is large enough already; a larger product then
+    replaces that workspace.  Every replay equals the product of the captured inputs."""
+    hip = _ffi.lib()                                          # (the HIP runtime's own functions, through the library that links it)
+
+    def call(f, *args):
+        assert getattr(hip, f)(*args) == 0, f
+
+    m, n, k = 64, 64, 777
+    rng = np.random.default_rng(5)
+    a, b = (rng.integers(-3, 4, s).astype(np.float32) for s in ((m, k), (k, n)))          # (integers: any order of the sums, the same bits)
+    bits = lambda x: (x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).ravel()
+    la, lb = np.ones((512, 8192)), np.ones((8192, 1024))
+    da, db, dla, dlb = (ctx.upload(bits(x)) for x in (a, b, la, lb))
+    dc, dlc = ctx.malloc(m * n * 4), ctx.malloc(512 * 1024 * 4)
+    desc = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), in_type=mz.IN_BF16, out_type=mz.OUT_F32)
+    larger = mz.gemm_ex_desc(mz.Matrix(dla, 512, 8192), mz.Matrix(dlb, 8192, 1024), mz.Matrix(dlc, 512, 1024), in_type=mz.IN_BF16, out_type=mz.OUT_F32)
+    s, graph, run = ctx.stream(), C.c_void_p(), C.c_void_p()
+    ctx.gemm_bf16(desc, s)
+    ctx.sync(s)
+    call("hipStreamBeginCapture", s, 1)
+    ctx.gemm_bf16(desc, s)
+    call("hipStreamEndCapture", s, C.byref(graph))
+    call("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+    for i in range(3):
+        dc.fill(0)
+        ctx.sync()
+        print(f"replay {i}", flush=True)
+        call("hipGraphLaunch", run, s)
+        ctx.sync(s)
+        assert np.array_equal(dc.download(np.float32).reshape(m, n), a @ b)
+        ctx.gemm_bf16(larger, s)
+        ctx.sync(s)
+        assert (dlc.download(np.float32) == 8192.0).all()
+    call("hipGraphExecDestroy", run)
+    call("hipGraphDestroy", graph)
+    ctx.stream_destroy(s)
+    for x in (da, db, dla, dlb, dc, dlc):
+        x.free()
