@@ -12,14 +12,14 @@ namespace {
 inline uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 inline uint64_t cdiv64(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
-// ---- maize_tile_*: tiles of 32 x 128, 64 x 64 and 64 x 128 (kernels/gemm_tile.hpp), fp32 also 128 x 128 -----------------
+// ---- maize_tile_*: tiles of 32 x 128, 64 x 64, 64 x 128 and (but for fp64) 128 x 128 (kernels/gemm_tile.hpp) -------------
 enum Tile : uint32_t { T32x128, T64x64, T64x128, T64x64W, T128x128, kTiles };     // W: 8-bit operands widened to bf16
 constexpr const char* const kOperands[8] = {"bf16", "f16", "e4m3", "e5m2", "e4m3e5m2", "e5m2e4m3", "f32", "f64"};   // maize_in_type_t's order
 constexpr uint32_t kTileForms = 8u * 2u * kTiles;
 static_assert(kTileForms <= kMaxForms, "the context's table of functions");
 bool tile_exists(uint32_t in_type, uint32_t tile) {
     const bool wide = in_type >= MAIZE_IN_F32;
-    return tile == T64x64W ? !wide && in_type >= MAIZE_IN_E4M3 : tile == T128x128 ? in_type == MAIZE_IN_F32 : true;
+    return tile == T64x64W ? !wide && in_type >= MAIZE_IN_E4M3 : tile == T128x128 ? in_type != MAIZE_IN_F64 : true;
 }
 struct Names {
     char name[kTileForms][40];
@@ -45,11 +45,15 @@ const Names& names() {
 // rows of A (B) that are no 16-byte material make the requests longer by ua (ub), transposing reads by nn, 8-bit
 // operands by e8; at least bytes / bw.
 struct TileCost { uint32_t bm, bn; double t0, one, many, turn, r0, r1, ua, ub, nn, bw, tail, e8; };
-constexpr TileCost kTileCost[T128x128] = {
+// 128 x 128 has a compute unit to itself and half of the LDS fill per product of 64 x 128: where its tiles make up one round or
+// few (129 to 256: 1024 x 3072 x 1999 into bf16 30.1 -> 24.5 us, 4499 x 520 x 3644 51.1 -> 35.8; below, K ranges of smaller tiles
+// keep the chip busier).  Fitted to 110 timings, residuals 7 % where it is a candidate.
+constexpr TileCost kTileCost[kTiles] = {
     {32, 128, 3.62, 0.215, 0.371, 0.0, 1.63, 0.14, 0.18, 0.36, 0.0, 6.55, 0.55, 0.07},
     {64, 64, 3.97, 0.167, 0.177, 1.06, 1.82, 0.19, 0.11, 0.40, 0.14, 6.88, 0.30, 0.10},
     {64, 128, 4.10, 0.278, 0.292, 1.49, 1.33, 0.54, 0.24, 0.25, 0.04, 6.03, 0.29, 0.09},
     {64, 64, 3.57, 0.329, 0.276, 1.27, 2.20, 0.22, 0.12, 0.15, 0.10, 5.21, 0.65, -0.04},
+    {128, 128, 4.42, 0.527, 0.527, 5.42, 0.0, 0.0, 0.14, 0.16, -0.05, 4.00, 1.50, -0.01},
 };
 // fp32 and fp64 operands: bound by the matrix instructions (a K tile of 64 x 64 is 1024 of their cycles, 0.43 us), so alignment
 // and layout cost next to nothing.  Fitted to 18600 timings of 1977 products, residuals 5-6 %.
@@ -176,7 +180,7 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     // best tile on four, by 3 % at most, and 4.3 times as long on average.
     const double rival = fam == kAnyShape || fam == kWide ? 1e9 : registry_cost(fam, p, ld.ksplit);
 
-    // The any-shape kernel multiplies 8-bit operands widened to bf16: its form does too.  Everywhere else the three tiles.
+    // The any-shape kernel multiplies 8-bit operands widened to bf16: its form does too.  Everywhere else the other tiles.
     const bool widened = bits8 && fam == kAnyShape;
     double best = 1e9;
     uint32_t tile = 0u, ranges = 1u;
@@ -194,8 +198,12 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
             // K ranges: of three K tiles or more, none empty, two workgroups per compute unit at most
             if (ks > 1u && (tiles * ks > (pinned ? 8u : 2u) * compute_units || p.steps / ks < 3u || t == T128x128)) break;
             if (ks > 1u && cdiv(p.steps, cdiv(p.steps, ks)) != ks) continue;
+            // (16- and 8-bit 128 x 128: from ten K tiles on and 8 % ahead of the others by the model: of 220 products 20 then run on it,
+            // 1.19x on average, one of them 3 % slower; without the two conditions up to 30 % slower, 413 deep)
+            const bool big = t == T128x128 && fam != kWide;
+            if (big && p.steps < 10u) break;
             const double cost = tile_cost(c, p, tiles, ks);
-            if (cost < best) { best = cost; tile = t; ranges = ks; }
+            if (cost < best * (big ? 0.92 : 1.0)) { best = cost; tile = t; ranges = ks; }
         }
     }
     // The form has to win 10 % by the model: of 590 products the choice is then 1.4 % behind the best of all candidates on

@@ -26,6 +26,11 @@
 // 3 x 4863 x 4281 48.6 -> 12.1, E4M3 19 x 10987 x 1494 50.1 -> 6.8; against the any-shape kernel: 150 x 201 x 333 26.1 -> 5.9, E4M3
 // 128 x 168 x 296 63 -> 5.5.  (Tried and slower: twice the ring depth on one workgroup per compute unit, three stages on three.)
 //
+// 128 x 128 of 16- and 8-bit operands: what bounds the smaller tiles on a product of a round or two is the LDS fill, which this
+// halves per multiply-add.  One workgroup of four ring stages (128 KiB) per compute unit: two of two stages have too few
+// registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
+// 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
+//
 // fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
 // What bounds them is the matrix pipe: a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
 // A lane's 16-byte chunk feeds four (two) instructions in turn, the same k on both sides, so a K-contiguous operand needs an
@@ -326,8 +331,8 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
         for (int j = 0; j < NJ; ++j) acc[i][j] = accx4{0, 0, 0, 0};
 
     // ---- the tail's loads, then the ring's first NS entries ----------------------------------------------------------
-    // (128 x 128: when they are placed, there are no registers to hold them through the loop)
-    constexpr bool LATE_TAIL = BM * BN > 64 * 128;
+    // (128 x 128 fp32: when they are placed, two workgroups per compute unit leave no registers to hold them through the loop)
+    constexpr bool LATE_TAIL = FP && BM * BN > 64 * 128;
     u32x4 ta[PA], tb[PB];
     auto load_tail = [&] {
 #pragma unroll
@@ -624,7 +629,9 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     MAIZE_TILE(maize_tile_##tag##_nn_32x128, et, false, false, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2)
+    MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 4, 1) \
+    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 4, 1)
 MAIZE_TILE_16(bf16, 0)
 MAIZE_TILE_16(f16, 1)
 #define MAIZE_TILE_8(tag, et) \
@@ -635,7 +642,9 @@ MAIZE_TILE_16(f16, 1)
     MAIZE_TILE(maize_tile_##tag##_nn_32x128, et, false, false, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2)
+    MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
+    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 4, 1) \
+    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 4, 1)
 MAIZE_TILE_8(e4m3, 2)
 MAIZE_TILE_8(e5m2, 5)
 MAIZE_TILE_8(e4m3e5m2, 4)

@@ -84,3 +84,34 @@ def test_form_kernels_keep_to_registers_and_plain_stores():
     assert len(names) >= 40
     for banned in ("scratch_", "v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32", "s_dcache_" + "wb", "s_sto" + "re", "s_ato" + "mic"):
         assert "\t" + banned not in text, banned
+
+
+@pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(HSACO)), reason="needs the ROCm llvm-objdump and the built code object")
+def test_no_register_that_a_fragment_read_is_still_filling_is_touched():
+    """The fragment reads are assembly statements, so the compiler takes their registers as written at once: where it runs out
+    of registers it may copy one before its data is there (128 x 128 tiles of 16-bit operands at two workgroups per compute
+    unit did, and gave wrong results).  Every kernel must wait first."""
+    text = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", HSACO], check=True, capture_output=True, text=True).stdout
+
+    def regs(s):
+        return {(kind, i) for kind, lo, hi, one in re.findall(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+)\b)", s)
+                for i in (range(int(lo), int(hi) + 1) if lo else [int(one)])}
+
+    kernel, filling, reads, early = None, set(), 0, []
+    for line in text.splitlines():
+        head = re.match(r"^[0-9a-f]+ <(maize_\w+)>:", line)
+        if head:
+            kernel, filling = head.group(1), set()
+        ins = re.match(r"^\t(\S+)\s*(.*?)\s*//", line)
+        if not ins:
+            continue
+        op, args = ins.groups()
+        if op == "s_waitcnt" and "lgkmcnt(0)" in args:
+            filling = set()
+        elif not op.startswith("s_"):
+            if regs(args) & filling:
+                early.append((kernel, line.split("//")[0].strip()))
+            if op.startswith("ds_read"):
+                reads += 1
+                filling |= regs(args.split(",")[0])
+    assert reads > 1000 and not early, early[:8]

@@ -84,7 +84,7 @@ def check_form(ctx, oracle, mod, op, tile, layout, m, n, k, ks=1, off=0, pad=0, 
 
 
 @pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
-@pytest.mark.parametrize("op,tile", [(op, t) for op in OPS for t in TILES if t != "128x128" and (op not in ("bf16", "f16") or t != "64x64w")])
+@pytest.mark.parametrize("op,tile", [(op, t) for op in OPS for t in TILES if (op not in ("bf16", "f16") or t != "64x64w")])
 def test_tile_forms_at_their_edges(ctx, oracle, forms, op, tile, layout):
     bm, bn = TILES[tile]
     kt = 64 if op in ("bf16", "f16") else 128
@@ -96,7 +96,7 @@ def test_tile_forms_at_their_edges(ctx, oracle, forms, op, tile, layout):
     check_form(ctx, oracle, forms, op, tile, layout, 2 * bm + 1, 9 * bn + 3, kt + 9, alpha=-1.25, beta=0.75)     # sweeps of 8 tile rows, ragged
     check_form(ctx, oracle, forms, op, tile, layout, 8 * bm + 5, 2 * bn - 1, kt, out_f32=True, alpha=0.5, beta=1.0, off=1)
     check_form(ctx, oracle, forms, op, tile, layout, bm + 1, bn + ch, 2 * kt + 5, batch=3, pad=1)
-    for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)):                                               # K ranges, the tail in the last
+    for ks, k in ((2, 9 * kt), (3, 9 * kt + 1), (16, 64 * kt - 7)) if tile != "128x128" else ():                  # K ranges, the tail in the last
         check_form(ctx, oracle, forms, op, tile, layout, bm + 3, bn + 5, k, ks=ks, out_f32=ks == 3)
 
 
