@@ -76,7 +76,21 @@ struct DeviceGuard {
 struct maize_workspace {
     void* ptr = nullptr;
     size_t bytes = 0;
+    bool in_graph = false;       // handed out while its stream was captured: a graph keeps the address
+    // Outgrown buffers that a graph keeps; they go with the stream.  Every buffer is more than 1.5 times its predecessor, so
+    // together they are less than twice the last one, and 64 of them are more than any device holds.
+    void* kept[64] = {};
+    uint32_t n_kept = 0;
 };
+// Frees a stream's buffers, those kept for graphs among them: the first error, if any.
+static hipError_t workspace_free(const maize_workspace& w) {
+    hipError_t e = w.ptr ? hipFree(w.ptr) : hipSuccess;
+    for (uint32_t i = 0; i < w.n_kept; ++i) {
+        const hipError_t ek = hipFree(w.kept[i]);
+        if (e == hipSuccess) e = ek;
+    }
+    return e;
+}
 struct maize_ctx {
     int device;
     hipDeviceProp_t prop;
@@ -195,8 +209,7 @@ int32_t maize_hip_ctx_destroy(maize_ctx_t* ctx) {
     if (!ctx) return fail(MAIZE_ERR_NULL, "ctx_destroy: ctx is NULL");
     DeviceGuard guard_;
     (void)guard_.enter(ctx->device);
-    for (auto& kv : ctx->workspaces)
-        if (kv.second.ptr) (void)hipFree(kv.second.ptr);
+    for (auto& kv : ctx->workspaces) (void)workspace_free(kv.second);
     hipError_t e = hipModuleUnload(ctx->module);
     const hipError_t ef = hipModuleUnload(ctx->forms_module);
     if (e == hipSuccess) e = ef;
@@ -459,20 +472,34 @@ int32_t maize_hip_gemm_select(maize_ctx_t* ctx, const maize_gemm_desc_t* desc, c
 // zero-filled (the ticket counters must start at zero; the kernels leave them at zero).
 static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void** out) {
     maize_workspace& w = ctx->workspaces[stream];
+    DeviceGuard guard_;
+    HIP_TRY(guard_.enter(ctx->device));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess)
+        (void)hipGetLastError();                             // (the null stream, while another one is captured: the launch reports it)
     if (w.bytes < bytes) {
-        DeviceGuard guard_;
-        HIP_TRY(guard_.enter(ctx->device));
-        if (w.ptr) {
+        if (w.ptr && !w.in_graph) {
             HIP_TRY(hipStreamSynchronize((hipStream_t)stream));  // earlier launches may still use the old one
             HIP_TRY(hipFree(w.ptr));
             w.ptr = nullptr;
             w.bytes = 0;
+        } else if (w.ptr && w.n_kept == sizeof w.kept / sizeof w.kept[0]) {
+            return fail(MAIZE_ERR_NOMEM, "gemm: too many workspaces kept for graphs");
         }
         const size_t want = bytes + bytes / 2;
-        HIP_TRY(hipMalloc(&w.ptr, want));
+        void* fresh;
+        HIP_TRY(hipMalloc(&fresh, want));
+        const hipError_t e = hipMemsetAsync(fresh, 0, want, (hipStream_t)stream);
+        if (e != hipSuccess) {
+            (void)hipFree(fresh);
+            return hip_fail(e, "hipMemsetAsync(workspace)");
+        }
+        if (w.ptr) w.kept[w.n_kept++] = w.ptr;
+        w.ptr = fresh;
         w.bytes = want;
-        HIP_TRY(hipMemsetAsync(w.ptr, 0, want, (hipStream_t)stream));
+        w.in_graph = false;
     }
+    w.in_graph |= capture != hipStreamCaptureStatusNone;
     *out = w.ptr;
     return MAIZE_OK;
 }
@@ -776,9 +803,9 @@ int32_t maize_hip_stream_destroy(maize_ctx_t* ctx, void* stream) {
     auto it = ctx->workspaces.find(stream);
     if (it != ctx->workspaces.end()) {
         HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
-        void* ws = it->second.ptr;
+        const maize_workspace ws = it->second;
         ctx->workspaces.erase(it);
-        if (ws) HIP_TRY(hipFree(ws));
+        HIP_TRY(workspace_free(ws));
     }
     HIP_TRY(hipStreamDestroy((hipStream_t)stream));
     return MAIZE_OK;

@@ -1,0 +1,126 @@
+"""The launcher (maize_amd/csrc/shim.cpp) on a model of the HIP runtime (tests/cpu/fake_hip.cpp): what it allocates, frees and
+launches, eagerly and while a stream is captured into a graph.  No device."""
+import ctypes as C
+import os
+import subprocess
+from types import SimpleNamespace
+
+import pytest
+
+import maize_amd as mz
+from maize_amd import _ffi
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "maize_amd", "csrc")
+STREAM, OTHER = C.c_void_p(0x1000), C.c_void_p(0x2000)
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    so = tmp_path_factory.mktemp("model") / "libmodel.so"
+    src = [os.path.join(CSRC, f) for f in ("shim.cpp", "dispatch.cpp", "forms.cpp")] + [os.path.join(ROOT, "tests", "cpu", "fake_hip.cpp")]
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-Wl,--no-undefined", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-o", str(so)] + src, check=True)
+    lib = C.CDLL(str(so))
+    lib.fake_log.restype = lib.maize_hip_last_error.restype = C.c_char_p
+    lib.fake_memory.argtypes = [C.c_size_t]
+    return lib
+
+
+class Device:
+    """One context on the model."""
+
+    def __init__(self, lib):
+        self.lib, self.ctx = lib, C.c_void_p()
+        lib.fake_memory(1 << 40)
+        assert lib.maize_hip_ctx_create(0, C.byref(self.ctx)) == 0
+        lib.fake_clear()
+
+    def close(self):
+        assert self.lib.maize_hip_ctx_destroy(self.ctx) == 0
+
+    def events(self):
+        """What was logged since the last call."""
+        out = []
+        for line in self.lib.fake_log().decode().splitlines():
+            w = line.split()
+            node = w[0] == "node"
+            w = w[node:]
+            if w[0] == "launch":
+                out.append(SimpleNamespace(what="launch", node=node, stream=int(w[1]), kernel=w[2], grid=int(w[3]), ksplit=int(w[4]), workspace=int(w[5])))
+            else:
+                out.append(SimpleNamespace(what=w[0], node=node, at=int(w[1]), rest=[int(x) for x in w[2:]]))
+        self.lib.fake_clear()
+        return out
+
+    def product(self, x, stream=STREAM):
+        rc = self.lib.maize_hip_gemm_bf16_ex(self.ctx, C.byref(x), None, stream)
+        assert rc == 0, (rc, self.lib.maize_hip_last_error())
+        return self.events()
+
+    def captured(self, x, stream=STREAM):
+        self.lib.fake_capture(stream)
+        ev = self.product(x, stream)
+        assert self.lib.fake_end_capture(stream) == 1, "the capture was spoilt"
+        return ev
+
+
+@pytest.fixture
+def dev(model):
+    d = Device(model)
+    yield d
+    d.close()
+
+
+def product(m, n, k, nt=False, in_type=mz.IN_BF16, batch=1, **how):
+    brows, bcols = (n, k) if nt else (k, n)
+    if batch > 1:
+        how.update(stride_a=m * k, stride_b=k * n, stride_c=m * n)
+    a, b, c = (mz.GlobalMatrix(p << 32, *s) for p, s in ((16, (m, k)), (32, (brows, bcols)), (48, (m, n))))
+    return mz.gemm_ex_desc(a, b, c, layout=mz.LAYOUT_NT if nt else mz.LAYOUT_NN, batch=batch, in_type=in_type, **how)
+
+
+def launches(events):
+    return [e for e in events if e.what == "launch"]
+
+
+# (the registry's kernel of the first needs scratch: it splits K; the second's needs none, its form 16.8 MB)
+FEW_ROWS, GROWS = product(16, 14336, 4096), product(267, 4320, 3648, nt=True)
+
+
+def test_a_buffer_that_a_graph_holds_is_not_freed_when_the_stream_needs_a_larger_one(dev):
+    dev.product(FEW_ROWS)
+    held = {e.workspace for e in launches(dev.captured(FEW_ROWS)) if e.workspace}
+    assert held
+    grown = dev.product(GROWS)
+    assert launches(grown)[0].ksplit > 1 and any(e.what == "malloc" for e in grown), "the larger product was meant to need a larger buffer"
+    assert not [e for e in grown if e.what == "free" and e.at in held]
+    # ... the eager product that follows is off the graph's buffer, and a graph taken now holds the larger one
+    assert not {e.workspace for e in launches(dev.product(FEW_ROWS))} & held
+    held |= {e.workspace for e in launches(dev.captured(FEW_ROWS))}
+    assert len(held) == 2
+    assert not [e for e in dev.product(product(512, 1024, 16384)) if e.what == "free" and e.at in held]
+
+
+def test_a_buffer_that_no_graph_holds_is_given_back(dev):
+    first = launches(dev.product(FEW_ROWS))[0].workspace
+    grown = dev.product(GROWS)
+    assert [e.what for e in grown][:3] == ["wait", "free", "malloc"] and grown[1].at == first
+
+
+def test_buffers_kept_for_graphs_go_with_the_stream_and_the_context(model):
+    for close in ("stream", "context"):
+        d = Device(model)
+        made = []
+        for stream in (STREAM, OTHER):
+            for x in (FEW_ROWS, GROWS):
+                made += [e.at for e in d.product(x, stream) if e.what == "malloc"]
+                d.captured(x, stream)
+        assert len(made) == 4
+        gone = []
+        if close == "stream":
+            assert model.maize_hip_stream_destroy(d.ctx, STREAM) == 0
+            gone = [e.at for e in d.events() if e.what == "free"]
+            assert sorted(gone) == made[:2]
+        d.close()
+        assert sorted(gone + [e.at for e in d.events() if e.what == "free"]) == made
