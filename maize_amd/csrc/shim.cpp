@@ -65,6 +65,14 @@ struct DeviceGuard {
     }
 };
 
+// While it lives the calling thread may allocate and free although a stream, of this thread or another, is being captured:
+// neither becomes part of a graph, and without this either would spoil the capture.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 #define HIP_TRY(expr)                                  \
     do {                                               \
         hipError_t e_ = (expr);                        \
@@ -77,8 +85,9 @@ struct maize_workspace {
     void* ptr = nullptr;
     size_t bytes = 0;
     bool in_graph = false;       // handed out while its stream was captured: a graph keeps the address
-    // Outgrown buffers that a graph keeps; they go with the stream.  Every buffer is more than 1.5 times its predecessor, so
-    // together they are less than twice the last one, and 64 of them are more than any device holds.
+    // Outgrown buffers that a graph keeps (or that a captured stream could not wait for); they go with the stream.  Every
+    // buffer is more than 1.5 times its predecessor, so together they are less than twice the last one, and 64 of them are
+    // more than any device holds.
     void* kept[64] = {};
     uint32_t n_kept = 0;
 };
@@ -468,8 +477,19 @@ int32_t maize_hip_gemm_select(maize_ctx_t* ctx, const maize_gemm_desc_t* desc, c
     return MAIZE_OK;
 }
 
+static hipError_t zero_now(void* p, size_t bytes) {
+    hipStream_t s;
+    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e != hipSuccess) return e;
+    e = hipMemsetAsync(p, 0, bytes, s);
+    const hipError_t es = hipStreamSynchronize(s), ed = hipStreamDestroy(s);
+    return e != hipSuccess ? e : es != hipSuccess ? es : ed;
+}
+
 // Returns the stream's workspace, grown to `bytes` if needed.  A new or grown workspace is
-// zero-filled (the ticket counters must start at zero; the kernels leave them at zero).
+// zero-filled (the ticket counters must start at zero; the kernels leave them at zero).  While the stream is captured that is
+// done at once on a stream of its own -- nothing but kernels is recorded, and eager launches may use the buffer before the
+// graph first runs -- and an old buffer, which the stream cannot be made to wait for, is kept.
 static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void** out) {
     maize_workspace& w = ctx->workspaces[stream];
     DeviceGuard guard_;
@@ -477,8 +497,10 @@ static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void*
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing((hipStream_t)stream, &capture) != hipSuccess)
         (void)hipGetLastError();                             // (the null stream, while another one is captured: the launch reports it)
+    const bool capturing = capture != hipStreamCaptureStatusNone;
     if (w.bytes < bytes) {
-        if (w.ptr && !w.in_graph) {
+        RelaxedCapture relaxed_;
+        if (w.ptr && !w.in_graph && !capturing) {
             HIP_TRY(hipStreamSynchronize((hipStream_t)stream));  // earlier launches may still use the old one
             HIP_TRY(hipFree(w.ptr));
             w.ptr = nullptr;
@@ -489,7 +511,7 @@ static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void*
         const size_t want = bytes + bytes / 2;
         void* fresh;
         HIP_TRY(hipMalloc(&fresh, want));
-        const hipError_t e = hipMemsetAsync(fresh, 0, want, (hipStream_t)stream);
+        const hipError_t e = capturing ? zero_now(fresh, want) : hipMemsetAsync(fresh, 0, want, (hipStream_t)stream);
         if (e != hipSuccess) {
             (void)hipFree(fresh);
             return hip_fail(e, "hipMemsetAsync(workspace)");
@@ -499,7 +521,7 @@ static int32_t workspace_for(maize_ctx_t* ctx, void* stream, size_t bytes, void*
         w.bytes = want;
         w.in_graph = false;
     }
-    w.in_graph |= capture != hipStreamCaptureStatusNone;
+    w.in_graph |= capturing;
     *out = w.ptr;
     return MAIZE_OK;
 }
@@ -596,9 +618,7 @@ static int32_t gemm_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, uint
                       sizeof args);
 }
 
-// Runs one of the launcher's own forms.  *ran = false: it cannot be run here, nothing was launched.  A form with K ranges
-// stays out of captured graphs: a graph keeps the address of the stream's workspace, which a later, larger product frees,
-// and the registry kernel may need none.
+// Runs one of the launcher's own forms.  *ran = false: it cannot be run here, nothing was launched.
 static int32_t form_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, const maize::FormPlan& f, void* stream,
                            const maize_workspace* fixed, bool* ran) {
     maize_gemm_args_t args = args_of(x);
@@ -608,12 +628,6 @@ static int32_t form_launch(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* x, cons
         if (f.workspace_bytes > fixed->bytes) return MAIZE_OK;
         args.workspace = fixed->ptr;
     } else if (f.workspace_bytes) {
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing((hipStream_t)stream, &capturing) != hipSuccess) {
-            (void)hipGetLastError();                                  // (the null stream, while another one is captured)
-            return MAIZE_OK;
-        }
-        if (capturing != hipStreamCaptureStatusNone) return MAIZE_OK;
         int32_t rc = workspace_for(ctx, stream, f.workspace_bytes, &args.workspace);
         if (rc != MAIZE_OK) return rc;
     }

@@ -124,3 +124,43 @@ def test_buffers_kept_for_graphs_go_with_the_stream_and_the_context(model):
             assert sorted(gone) == made[:2]
         d.close()
         assert sorted(gone + [e.at for e in d.events() if e.what == "free"]) == made
+
+
+def route(events):
+    return [(e.kernel, e.grid, e.ksplit) for e in launches(events)]
+
+
+# a form in K ranges where the registry's kernel wants more scratch (packed copies), wants none, or is its twin; one without
+# K ranges; a registry kernel in K ranges; and one with a reduce pass behind it
+CAPTURED = [product(64, 64, 1999), GROWS, product(3, 4863, 4281), product(8, 7336, 4464, in_type=mz.IN_F32), product(150, 201, 333), FEW_ROWS, product(2048, 2048, 16384)]
+
+
+@pytest.mark.parametrize("x", CAPTURED)
+def test_a_captured_call_runs_what_the_eager_call_runs(model, x):
+    """... with the same workspace where the stream has run it before, and with one of its own, zero before the graph first
+    runs and not set by it, where it has not.  Neither spoils the capture."""
+    warm, cold = Device(model), Device(model)
+    eager = warm.product(x)
+    again = warm.captured(x)
+    assert route(again) == route(eager) and [e.what for e in again] == ["launch"] * len(again)
+    assert [e.workspace for e in launches(again)] == [e.workspace for e in launches(eager)]
+    first = cold.captured(x)
+    assert route(first) == route(eager) and not model.fake_relaxed()
+    for e in first:
+        assert e.node == (e.what == "launch")
+        if e.what == "set":
+            assert e.at != STREAM.value and [f.at for f in first if f.what == "wait"] == [e.at]
+    assert route(cold.product(x)) == route(eager)
+    # grown within a capture: what earlier launches and the graph use stays
+    cold.product(product(64, 64, 1999), OTHER)
+    grown = cold.captured(x, OTHER)
+    assert route(grown) == route(eager) and not [e for e in grown if e.what == "free"]
+    warm.close()
+    cold.close()
+
+
+def test_growing_a_workspace_does_not_spoil_the_capture_of_another_stream(dev, model):
+    model.fake_capture(OTHER)
+    dev.product(FEW_ROWS)
+    assert any(e.what == "free" for e in dev.product(GROWS))
+    assert model.fake_end_capture(OTHER) == 1 and not model.fake_relaxed()
