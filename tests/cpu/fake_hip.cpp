@@ -73,7 +73,7 @@ const char* hipGetErrorString(hipError_t) { return "error of the model"; }
 hipError_t hipGetLastError() { const hipError_t e = g_last; g_last = hipSuccess; return e; }
 hipError_t hipMalloc(void** p, size_t n) {
     if (unsafe_call()) return ret(hipErrorStreamCaptureUnsupported);
-    if (n > g_limit - g_used) return ret(hipErrorOutOfMemory);
+    if (g_used + n > g_limit) return ret(hipErrorOutOfMemory);
     *p = (void*)g_next;
     g_live[g_next] = n;
     say("malloc %" PRIu64 " %zu\n", g_next, n);
@@ -108,7 +108,7 @@ hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
     return hipSuccess;
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) { std::swap(*m, g_mode); return hipSuccess; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)g_next++; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)g_next; g_next += 0x10000; return hipSuccess; }
 hipError_t hipStreamCreate(hipStream_t* s) { return hipStreamCreateWithFlags(s, 0); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipModuleLoadData(hipModule_t* m, const void*) { *m = (hipModule_t)1; return hipSuccess; }

@@ -164,3 +164,15 @@ def test_growing_a_workspace_does_not_spoil_the_capture_of_another_stream(dev, m
     dev.product(FEW_ROWS)
     assert any(e.what == "free" for e in dev.product(GROWS))
     assert model.fake_end_capture(OTHER) == 1 and not model.fake_relaxed()
+
+
+def test_a_product_whose_kernel_needs_no_device_memory_runs_when_there_is_none(dev, model):
+    want = route(dev.product(GROWS))
+    assert want[0][2] > 1                                        # a form in K ranges ...
+    model.fake_memory(0)
+    ran = launches(dev.product(GROWS, OTHER))
+    assert len(ran) == 1 and ran[0].kernel == mz.gemm_plan(GROWS)["kernel"] and ran[0].workspace == 0
+    assert model.hipGetLastError() == 0
+    # ... one whose kernel needs scratch as well is an error, as it is for a kernel that is named
+    assert model.maize_hip_gemm_bf16_ex(dev.ctx, C.byref(product(64, 64, 1999)), None, OTHER) == 2
+    assert not launches(dev.events())
