@@ -193,7 +193,8 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
         if ((t == T64x64W) != widened || !tile_exists(d.in_type, t)) continue;
         const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][t] : kTileCost[t];
         const uint64_t tiles = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch;
-        if (tiles > (1u << 24) || (t == T32x128 && p.s.m > 96u)) continue;
+        // (a launch counts its work items in 32 bits: fewer than 2^24 workgroups of 256)
+        if (tiles >= (1u << 24) || (t == T32x128 && p.s.m > 96u)) continue;
         for (uint32_t ks = ks_lo; ks <= ks_hi; ++ks) {
             // K ranges: of three K tiles or more, none empty, two workgroups per compute unit at most
             if (ks > 1u && (tiles * ks > (pinned ? 8u : 2u) * compute_units || p.steps / ks < 3u || t == T128x128)) break;

@@ -176,3 +176,10 @@ def test_a_product_whose_kernel_needs_no_device_memory_runs_when_there_is_none(d
     # ... one whose kernel needs scratch as well is an error, as it is for a kernel that is named
     assert model.maize_hip_gemm_bf16_ex(dev.ctx, C.byref(product(64, 64, 1999)), None, OTHER) == 2
     assert not launches(dev.events())
+
+
+@pytest.mark.parametrize("x", [product(32768, 8, 9, batch=32768), product(1, 65536, 64, batch=32768, in_type=mz.IN_F32), product(32, 128, 64, batch=65535, in_type=mz.IN_F32),
+                               product(4095 * 64, 64, 64, batch=4096, in_type=mz.IN_E4M3)])
+def test_a_launch_stays_within_32_bits_of_work_items(dev, x):
+    """Tiles that would make up 2^24 workgroups of 256, and a little fewer: the product runs, in a grid that a launch can have."""
+    assert launches(dev.product(x))                              # (the model refuses what the runtime refuses)
