@@ -25,9 +25,15 @@
  *  - Kernels that split K or repack operands use a workspace the library owns,
  *    one per (context, stream), allocated (or grown) by the first launch that
  *    needs it: that launch calls hipMalloc and, when growing, waits for the
- *    stream.  maize_hip_gemm_plan reports the bytes.  The workspace is released
+ *    stream.  maize_hip_gemm_ex_form reports the bytes, or maize_hip_gemm_plan
+ *    where no form runs or a kernel is named.  The workspace is released
  *    by maize_hip_stream_destroy for streams made by maize_hip_stream_create,
  *    and by maize_hip_ctx_destroy for every other stream it was used with.
+ *  - A stream may be captured into a graph: the same kernels are recorded as
+ *    are launched eagerly, and nothing else.  A workspace that a graph uses is
+ *    kept until the stream's workspace is released, also when a larger product
+ *    replaces it; a graph must not be replayed after that, nor while other work
+ *    of its stream is in flight on another one.
  *  - Arithmetic: products of bf16 operands are exact, sums are kept in fp32 (one rounding per 16- or 32-deep matrix
  *    instruction), C is rounded once to bf16 (nearest even).  IEEE special values follow through: NaN and +-Inf in A or
  *    B give NaN / Inf exactly where an fp64 evaluation does (the zero fill of the M, N and K edges never meets a real
@@ -231,13 +237,15 @@ uint32_t maize_hip_get_split_wait_us(void);
  * fails with MAIZE_ERR_KERNEL if that kernel cannot run the descriptor. */
 int32_t maize_hip_gemm_bf16_with(maize_ctx_t* ctx, const maize_gemm_desc_t* desc,
                                  const char* kernel, void* stream);
-/* Which kernel maize_hip_gemm_bf16 would pick; writes a NUL-terminated name.  (What this and maize_hip_gemm_plan report is the
- * registry's choice.  Where no kernel is named the launcher may run one of its own forms in its place -- small tiles for any
- * alignment, maize_amd/csrc/forms.hpp -- with the same operand handling and accuracy.  Naming the kernel runs exactly it.) */
+/* Which registry kernel maize_hip_gemm_bf16 would pick; writes a NUL-terminated name.  (What this and maize_hip_gemm_plan report
+ * is the registry's choice.  Where no kernel is named the launcher may run one of its own forms in its place -- small tiles for
+ * any alignment, maize_amd/csrc/forms.hpp -- with the same operand handling and accuracy: maize_hip_gemm_ex_form tells.  Naming
+ * the kernel runs exactly it.) */
 int32_t maize_hip_gemm_select(maize_ctx_t* ctx, const maize_gemm_desc_t* desc, char* name, size_t cap);
 /* Launch geometry for `desc` on a device with `compute_units` compute units (no device access):
- * which kernel (`kernel` == NULL: the dispatcher's choice), its grid and block, the number of K
- * ranges of a split kernel and the bytes of library-owned workspace the launch uses.  This is
+ * which registry kernel (`kernel` == NULL: the dispatcher's choice), its grid and block, the number of K
+ * ranges of a split kernel and the bytes of library-owned workspace its launch uses (with `kernel` == NULL the
+ * launcher may run a form in its place: maize_hip_gemm_ex_form).  This is
  * the decision the reference's panel iterators make when they turn extents and a grid into
  * per-block work (crates/maize_tile/src/gmem/row_panel.rs:85-127, col_panel.rs:88-124). */
 typedef struct {
@@ -272,6 +280,11 @@ int32_t maize_hip_gemm_ex_tail_rows(const maize_gemm_ex_desc_t* desc, uint32_t c
  * reports 0 for a product cut by columns.  16-bit and 8-bit operands (E4M3 4352 x 4096 x 4096: 79.8 -> 66.3 us); batches and
  * fp32 / fp64 operands are always one product.  No counterpart in the reference (see above). */
 int32_t maize_hip_gemm_ex_tail_split(const maize_gemm_ex_desc_t* desc, uint32_t compute_units, uint32_t* rows, uint32_t* cols);
+/* What the launcher runs with kernel == NULL where that is not the kernel gemm_ex_plan names: one of its own forms (kernels
+ * maize_tile_*, maize_amd/csrc/forms.hpp), with its grid, K ranges and workspace.  out->kernel == "" (all else 0): it runs what
+ * gemm_ex_plan and gemm_ex_tail_split describe.  The form gives way to that kernel where its workspace cannot be had (no device
+ * memory).  A form is not a registry kernel: it cannot be named in a call.  No counterpart in the reference. */
+int32_t maize_hip_gemm_ex_form(const maize_gemm_ex_desc_t* desc, uint32_t compute_units, maize_gemm_plan_t* out);
 /* Validation only (no device access): the checks gemm_bf16 performs first. */
 int32_t maize_hip_gemm_validate(const maize_gemm_desc_t* desc);
 /* Enumerates the GEMM kernels of the embedded code object. */

@@ -248,16 +248,32 @@ def gemm_plan(desc, kernel=None, compute_units=256):
     out = _ffi.GemmPlanT()
     fn = _ffi.lib().maize_hip_gemm_ex_plan if isinstance(desc, _ffi.GemmExDescT) else _ffi.lib().maize_hip_gemm_plan
     check(fn(C.byref(desc), kernel.encode() if kernel else None, compute_units, C.byref(out)))
+    return _plan_dict(out)
+
+
+def _plan_dict(out):
     return {"kernel": out.kernel.decode(), "grid": tuple(out.grid), "block": tuple(out.block), "lds_bytes": out.lds_bytes,
             "ksplit": out.ksplit, "split_first": out.split_first, "reduce_grid": out.reduce_grid,
             "workspace_bytes": out.workspace_bytes}
 
 
+def _extended(desc):
+    return desc if isinstance(desc, _ffi.GemmExDescT) else gemm_ex_desc(desc.a, desc.b, desc.c, layout=desc.layout, batch=desc.batch,
+                                                                        stride_a=desc.stride_a, stride_b=desc.stride_b, stride_c=desc.stride_c)
+
+
+def gemm_form(desc, compute_units=256):
+    """The form that the launcher runs in place of the kernel that ``gemm_plan`` reports, where no kernel is named: a dict like
+    its, or None (no device needed)."""
+    out = _ffi.GemmPlanT()
+    check(_ffi.lib().maize_hip_gemm_ex_form(C.byref(_extended(desc)), compute_units, C.byref(out)))
+    return _plan_dict(out) if out.kernel else None
+
+
 def gemm_tail_rows(desc, compute_units=256):
     """Leading rows of A and C the launcher computes as a product of their own when the tile count is a little over
     a whole number of rounds (the rest follows as a second, split-K product); 0 = one product.  No device needed."""
-    x = desc if isinstance(desc, _ffi.GemmExDescT) else gemm_ex_desc(desc.a, desc.b, desc.c, layout=desc.layout, batch=desc.batch,
-                                                                      stride_a=desc.stride_a, stride_b=desc.stride_b, stride_c=desc.stride_c)
+    x = _extended(desc)
     rows = C.c_uint32()
     check(_ffi.lib().maize_hip_gemm_ex_tail_rows(C.byref(x), compute_units, C.byref(rows)))
     return rows.value
@@ -266,8 +282,7 @@ def gemm_tail_rows(desc, compute_units=256):
 def gemm_tail_split(desc, compute_units=256):
     """(rows, cols): how the launcher cuts a product whose tile count is a little over a whole number of rounds -- the
     leading rows first, or the leading columns first, the rest behind them as a product of its own; (0, 0) = one product."""
-    x = desc if isinstance(desc, _ffi.GemmExDescT) else gemm_ex_desc(desc.a, desc.b, desc.c, layout=desc.layout, batch=desc.batch,
-                                                                      stride_a=desc.stride_a, stride_b=desc.stride_b, stride_c=desc.stride_c)
+    x = _extended(desc)
     rows, cols = C.c_uint32(), C.c_uint32()
     check(_ffi.lib().maize_hip_gemm_ex_tail_split(C.byref(x), compute_units, C.byref(rows), C.byref(cols)))
     return rows.value, cols.value

@@ -412,6 +412,33 @@ int32_t maize_hip_gemm_ex_tail_split(const maize_gemm_ex_desc_t* desc, uint32_t 
     return MAIZE_OK;
 }
 
+// The launcher's choice where no kernel is named: the registry's, and whether one of the forms runs in its place.
+static int32_t choose(const maize_gemm_ex_desc_t& x, uint32_t cus, uint32_t* registry, maize::FormPlan* form, bool* has_form) {
+    const int32_t rc = select_checked(x, cus, registry);
+    *has_form = rc == MAIZE_OK && maize::choose_form(x, *registry, cus, form);
+    return rc;
+}
+
+int32_t maize_hip_gemm_ex_form(const maize_gemm_ex_desc_t* desc, uint32_t compute_units, maize_gemm_plan_t* out) {
+    if (!out) return fail(MAIZE_ERR_NULL, "gemm_form: NULL argument");
+    int32_t rc = maize_hip_gemm_ex_validate(desc);
+    if (rc != MAIZE_OK) return rc;
+    if (compute_units == 0) return fail(MAIZE_ERR_ARG, "gemm_form: compute_units must be positive");
+    uint32_t registry;
+    maize::FormPlan f;
+    bool has_form;
+    if ((rc = choose(*desc, compute_units, &registry, &f, &has_form)) != MAIZE_OK) return rc;
+    memset(out, 0, sizeof(*out));
+    if (!has_form) return MAIZE_OK;
+    snprintf(out->kernel, sizeof(out->kernel), "%s", maize::form_name(f.kernel));
+    out->grid[0] = f.grid;
+    out->block[0] = 256;
+    out->grid[1] = out->grid[2] = out->block[1] = out->block[2] = 1;
+    out->ksplit = f.ksplit;
+    out->workspace_bytes = f.workspace_bytes;
+    return MAIZE_OK;
+}
+
 const char* maize_hip_kernel_name(uint32_t index) {
     return index < maize::kernel_count() ? maize::kernel_at(index).name : nullptr;
 }
@@ -661,11 +688,12 @@ static int32_t gemm_ex(maize_ctx_t* ctx, const maize_gemm_ex_desc_t* desc, const
     if (!kernel) {
         const uint32_t cus = (uint32_t)ctx->prop.multiProcessorCount;
         uint32_t chosen;
-        if ((rc = select_checked(*desc, cus, &chosen)) != MAIZE_OK) return rc;
+        maize::FormPlan form;
+        bool has_form;
+        if ((rc = choose(*desc, cus, &chosen, &form, &has_form)) != MAIZE_OK) return rc;
         // One of the launcher's own forms, where it is faster (fixed scratch: what the registry's plan does not fit is refused
         // all the same, as documented).
-        maize::FormPlan form;
-        if (maize::choose_form(*desc, chosen, cus, &form)) {
+        if (has_form) {
             bool ran;
             if (fixed && (rc = fits_fixed(ctx, desc, chosen, fixed)) != MAIZE_OK) return rc;
             rc = form_launch(ctx, desc, form, stream, fixed, &ran);

@@ -183,3 +183,21 @@ def test_a_product_whose_kernel_needs_no_device_memory_runs_when_there_is_none(d
 def test_a_launch_stays_within_32_bits_of_work_items(dev, x):
     """Tiles that would make up 2^24 workgroups of 256, and a little fewer: the product runs, in a grid that a launch can have."""
     assert launches(dev.product(x))                              # (the model refuses what the runtime refuses)
+
+
+# products that a form takes -- every tile, one K range and several, widened 8-bit operands, fp32 and fp64 -- and two that none takes
+DESCRIBED = CAPTURED + [product(64, 64, 64), product(200, 1072, 368), product(544, 2472, 1112), product(1024, 3072, 1999), product(9, 2304, 2048), product(16, 14336, 4096, nt=True, in_type=mz.IN_E4M3),
+                        product(128, 168, 296, in_type=mz.IN_E5M2_E4M3), product(1000, 1000, 1000, in_type=mz.IN_F64), product(1024, 4096, 4096, nt=True)]
+
+
+@pytest.mark.parametrize("x", DESCRIBED)
+def test_form_query_describes_the_launch(dev, x):
+    form, plan, ran = mz.gemm_form(x), mz.gemm_plan(x), dev.product(x)
+    first, bytes_ = launches(ran)[0], [e.rest[0] for e in ran if e.what == "malloc"]
+    want = form or plan
+    assert bytes_ == ([want["workspace_bytes"] * 3 // 2] if want["workspace_bytes"] else [])
+    if form:
+        assert (first.kernel, first.grid, max(1, first.ksplit)) == (form["kernel"], form["grid"][0], form["ksplit"])
+        assert form["grid"][1:] == (1, 1) and form["block"] == (256, 1, 1) and len(launches(ran)) == 1
+    else:
+        assert first.grid == plan["grid"][0] * plan["grid"][1] * plan["grid"][2]
