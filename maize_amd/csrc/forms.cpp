@@ -210,6 +210,12 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     // The form has to win 10 % by the model: of 590 products the choice is then 1.4 % behind the best of all candidates on
     // average, and six are slower than with the registry kernel alone, by 3 to 19 % (none allowed: 1.86x on average, all: 1.855x).
     if (best >= 0.9 * rival) return false;
+    // A product that the launcher would cut was compared with its uncut kernel only: it stays cut (4453 x 3712 x 2432 71 us against
+    // 79 on the form, 816 x 18448 x 11456 320 against 465, E4M3 1387 x 11200 x 15040 214 against 316).
+    if (fam == kMT256 && cdiv64((uint64_t)cdiv(p.s.m, 256) * cdiv(p.s.n, 256), compute_units) > 1u) {
+        const TailSplit cut = tail_split(d, compute_units);
+        if (cut.rows || cut.cols) return false;
+    }
     const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][tile] : kTileCost[tile];
     const uint64_t items = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch * ranges;
     out->kernel = (d.in_type * 2u + (p.s.nt ? 1u : 0u)) * kTiles + tile;
