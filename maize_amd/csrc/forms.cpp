@@ -76,67 +76,90 @@ struct Problem {
     Dims s;
     uint32_t batch, esz, bke, steps, cus;    // bytes per element of A and B; elements and number of K tiles
     bool rows_a, rows_b, tail;               // rows that are 16-byte material; a ragged last K tile
-    double bytes;                            // each operand once
+    double bytes, ab_bytes;                  // each operand once; A and B alone
 };
-double tile_cost(const TileCost& c, const Problem& p, uint64_t tiles, uint32_t ks) {
+double tile_cost(const TileCost& c, const Problem& p, uint64_t tiles, uint32_t ks, double wait = 1.0) {
     const uint32_t per = cdiv(p.steps, ks);
     const double items = (double)(tiles * ks), each = (p.rows_a ? 1.0 : 1.0 + c.ua) * (p.rows_b ? 1.0 : 1.0 + c.ub) * (p.s.nt ? 1.0 : 1.0 + c.nn) * (p.esz == 1u ? 1.0 + c.e8 : 1.0);
     const uint64_t n = cdiv64(tiles * ks, p.cus);
-    const double core = n <= 1u ? per * c.one * each : per * c.many * each * (n > 6u ? items / p.cus : (double)n) + c.turn * (double)(n - 1u);
+    const double core = wait * (n <= 1u ? per * c.one * each : per * c.many * each * (n > 6u ? items / p.cus : (double)n)) + c.turn * (double)(n - 1u);
     return c.t0 + longer(core, p.bytes / (c.bw * 1e6)) + (p.tail ? c.tail : 0.0) + (ks > 1u ? c.r0 + c.r1 * ks : 0.0);
 }
-
-// The registry's kernels, by what their time depends on.  The same fit, of the time of the call (kernel, copies and reduce
-// pass) on the same products: one coefficient set per family, residuals 8-23 %.
-enum Family : uint32_t { kSkinnyNN, kSkinnyNT, kCopies, kT128, kH128, kH128R3, kMT256, kH128Split, kMT256Split, kAnyShape, kWide };
-Family family_of(const char* name) {
-    if (std::strstr(name, "_mt128_")) return kWide;
-    if (std::strstr(name, "_wave32")) return kAnyShape;
-    if (std::strstr(name, "_skinny_nn")) return kSkinnyNN;
-    if (std::strstr(name, "_skinny_nt")) return kSkinnyNT;
-    if (std::strstr(name, "_packed") || std::strstr(name, "_trb")) return kCopies;
-    if (std::strstr(name, "_t128_")) return kT128;
-    if (std::strstr(name, "_splitk")) return std::strstr(name, "_h128") ? kH128Split : kMT256Split;
-    return std::strstr(name, "_h128r3") ? kH128R3 : std::strstr(name, "_h128") ? kH128 : kMT256;
+// Operands that the eight L2s (32 MB together) do not hold make a K tile wait longer: core * (their bytes / 32 MB)^0.18, ^0.085 for
+// 128 x 128 tiles, which draw half as much (fitted to 3568 timings, up to 2.1 times the model's without).  It decides between a
+// form and the registry's kernel (but for few rows, bound by the stream of B either way), not between forms, where it costs as much
+// as it gives on some products.
+double wait_factor(const TileCost& c, const Problem& p) {
+    return p.ab_bytes > 32e6 ? std::pow(p.ab_bytes / 32e6, c.bm == 128u ? 0.085 : 0.18) : 1.0;
 }
-const Family* families() {
+
+// The registry's kernels, by what their time depends on.
+enum Family : uint32_t { kSkinnyNN, kSkinnyNT, kPacked, kPackedGen, kTransposed, kT128, kH128, kH128Gen, kH128R3, kH128R3Gen, kMT256, kMT256Gen, kH128Split, kMT256Split,
+                         kAnyShape, kWide, kUnknown };
+struct FamilyOf { Family family; bool whole_m, whole_n; };      // whole_*: a narrow last tile row (column) rides along or is split
+FamilyOf family_of(const char* name) {
+    const auto has = [&](const char* part) { return std::strstr(name, part) != nullptr; };
+    if (has("_mt128_")) return {kWide, false, false};
+    if (has("_wave32")) return {kAnyShape, false, false};
+    if (has("_skinny_nn")) return {kSkinnyNN, false, false};
+    if (has("_skinny_nt")) return {kSkinnyNT, false, false};
+    if (has("_packed_gen")) return {kPackedGen, false, false};
+    if (has("_packed")) return {kPacked, false, false};
+    if (has("_trb")) return {kTransposed, false, false};
+    if (has("_t128_")) return {kT128, false, false};
+    if (!has("_mt256_")) return {kUnknown, false, false};
+    if (has("_splitk")) return {has("_h128") ? kH128Split : kMT256Split, false, false};
+    const bool gen = has("_gen");                                    // (the general epilogue)
+    if (has("_h128")) return {has("_h128r3") ? (gen ? kH128R3Gen : kH128R3) : gen ? kH128Gen : kH128, false, false};
+    return {gen ? kMT256Gen : kMT256, has("_edge") || has("_ragged_m"), has("_edge") || (has("_ragged") && !has("_ragged_m"))};
+}
+const FamilyOf* families() {
     struct Table {
-        Family of[kMaxKernels];
+        FamilyOf of[kMaxKernels];
         Table() { for (uint32_t i = 0; i < kernel_count(); ++i) of[i] = family_of(kernel_at(i).name); }
     };
     static const Table t;
     return t.of;
 }
-// t0, per K tile and round, per further round, per Mi elements of C (and round), per K range, per K range and Mi elements, 8-bit.
-struct TiledCost { uint32_t bm, bn; double t0, step, round, c, range, crange, e8; };
-double tiled_cost(const TiledCost& c, const Problem& p, uint32_t ks) {
-    const double elems = (double)p.s.m * p.s.n * p.batch * 1e-6;
-    const double rounds = (double)cdiv64((uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch * ks, p.cus);
-    const double core = rounds * cdiv(p.steps, ks) * c.step * (p.esz == 1u ? 1.0 + c.e8 : 1.0) + (rounds - 1.0) * c.round;
-    return c.t0 + longer(core, p.bytes / 4.6e6) + c.c * elems / rounds + (c.range + c.crange * elems) * ks;
-}
-double registry_cost(Family f, const Problem& p, uint32_t ks) {
-    if (ks == 0u) ks = 1u;
-    switch (f) {
-        case kSkinnyNN: case kSkinnyNT: {
-            const bool nn = f == kSkinnyNN;
-            const uint32_t groups = p.s.m <= 16u ? 1u : p.s.m <= 32u ? 2u : 4u;
-            const double rounds = (double)cdiv64((uint64_t)cdiv(p.s.n, 256) * p.batch * ks, p.cus);
-            const double core = rounds * cdiv(p.steps, ks) * (nn ? 0.44 : 0.85);
-            return (nn ? 3.5 : 1.0) + longer(core, p.bytes / (nn ? 6.35e6 : 5.33e6)) + (ks > 1u ? (nn ? 3.8 : 0.0) + (nn ? 0.19 : 0.65) * ks * groups : 0.0);
-        }
-        case kCopies: {
-            const double rounds = (double)cdiv64((uint64_t)cdiv(p.s.m, 256) * cdiv(p.s.n, 256) * p.batch * ks, p.cus);
-            return 16.5 + rounds * cdiv(p.steps, ks) * 1.175 + 0.69e-6 * p.batch * p.esz * ((double)p.s.m + p.s.n) * p.s.k + 2.07e-6 * p.s.m * p.s.n * p.batch * ks;
-        }
-        case kT128:       return tiled_cost({128, 128, 4.6, 0.385, 7.1, 0.2, 0.0, 0.0, 0.0}, p, 1u);
-        case kH128:       return tiled_cost({128, 256, 5.3, 0.63, 12.0, 0.4, 0.0, 0.0, 0.45}, p, 1u);
-        case kH128R3:     return tiled_cost({128, 256, 2.75, 0.775, 7.1, 0.52, 0.0, 0.0, 0.07}, p, 1u);
-        case kMT256:      return tiled_cost({256, 256, 6.9, 1.27, 4.4, 0.06, 0.0, 0.0, 0.08}, p, 1u);
-        case kH128Split:  return tiled_cost({128, 256, 6.6, 0.73, 8.8, 0.0, 0.37, 1.42, 0.07}, p, ks);
-        case kMT256Split: return tiled_cost({256, 256, 6.8, 1.68, 12.0, 0.33, 0.0, 1.8, 0.0}, p, ks);
-        default:          return 1e9;
+// The time of the call (kernel, copies and reduce pass), microseconds: t0 + rounds (step * K tiles of a range + round) +
+// (c + crange * ranges) 10^6 elements of C + range * ranges + mb * MB of A and B + copy * MB copied first.  Fitted to the timings
+// of 8630 products (operands cycled): medians of measured over fitted 1.00-1.05, the 5th and 95th percentiles 0.84-0.94 and
+// 1.08-1.34.  Rows: 16-bit and 8-bit operands.
+struct RegistryCost { uint32_t bm, bn; double t0, step, round, c, range, crange, mb, copy; };
+constexpr RegistryCost kRegistryCost[kAnyShape][2] = {
+    {}, {},                                                                                                                         // (few rows: below)
+    {{256, 256, 10.7, 1.21, 3.45, 0.757, 0.274, 1.33, 0.0, 0.673}, {256, 256, 11.8, 1.21, 5.47, 0.987, 0.141, 0.859, 0.0, 1.34}},   // kPacked
+    {{256, 256, 10.3, 1.12, 3.56, 0.427, 0.0, 0.0, 0.0, 0.652}, {256, 256, 11.8, 1.21, 5.47, 0.987, 0.141, 0.859, 0.0, 1.34}},      // kPackedGen
+    {{}, {256, 256, 7.86, 1.33, 1.85, 0.536, 0.0, 0.0, 0.0, 0.983}},                                                                // kTransposed
+    {{128, 128, 4.09, 0.363, 0.0, 0.56, 0.0, 0.0, 0.037, 0.0}, {128, 128, 4.2, 0.359, 0.0, 0.563, 0.0, 0.0, 0.002, 0.0}},           // kT128
+    {{128, 256, 0.0, 0.554, 3.89, 0.348, 0.0, 0.0, 0.104, 0.0}, {}},                                                                // kH128
+    {{128, 256, 0.0, 0.765, 4.67, 0.821, 0.0, 0.0, 0.061, 0.0}, {128, 256, 0.0, 0.705, 5.27, 0.74, 0.0, 0.0, 0.009, 0.0}},          // kH128Gen
+    {{128, 256, 0.0, 0.633, 0.0, 0.867, 0.0, 0.0, 0.058, 0.0}, {}},                                                                 // kH128R3
+    {{128, 256, 0.0, 0.819, 1.33, 1.02, 0.0, 0.0, 0.042, 0.0}, {128, 256, 0.0, 0.724, 1.8, 0.913, 0.0, 0.0, 0.054, 0.0}},           // kH128R3Gen
+    {{256, 256, 2.4, 1.29, 3.47, 0.177, 0.0, 0.0, 0.055, 0.0}, {256, 256, 3.36, 1.17, 3.59, 0.192, 0.0, 0.0, 0.055, 0.0}},          // kMT256
+    {{256, 256, 3.88, 1.4, 5.23, 0.226, 0.0, 0.0, 0.042, 0.0}, {256, 256, 3.36, 1.17, 3.59, 0.192, 0.0, 0.0, 0.055, 0.0}},          // kMT256Gen
+    {{128, 256, 0.0, 0.537, 6.49, 2.16, 0.318, 1.51, 0.076, 0.0}, {128, 256, 0.0, 0.435, 6.93, 2.27, 0.314, 1.62, 0.05, 0.0}},      // kH128Split
+    {{256, 256, 6.13, 1.4, 1.59, 1.23, 0.379, 1.06, 0.047, 0.0}, {256, 256, 0.0, 1.4, 5.99, 2.68, 0.0, 0.535, 0.053, 0.0}},         // kMT256Split
+};
+double registry_cost(const FamilyOf& f, const Problem& p, const LaunchDims& ld) {
+    const uint32_t ks = ld.ksplit ? ld.ksplit : 1u;
+    if (f.family == kSkinnyNN || f.family == kSkinnyNT) {
+        const bool nn = f.family == kSkinnyNN;
+        const uint32_t groups = p.s.m <= 16u ? 1u : p.s.m <= 32u ? 2u : 4u;
+        const double rounds = (double)cdiv64((uint64_t)cdiv(p.s.n, 256) * p.batch * ks, p.cus);
+        const double core = rounds * cdiv(p.steps, ks) * (nn ? 0.44 : 0.85);
+        return (nn ? 3.5 : 1.0) + longer(core, p.bytes / (nn ? 6.35e6 : 5.33e6)) + (ks > 1u ? (nn ? 3.8 : 0.0) + (nn ? 0.19 : 0.65) * ks * groups : 0.0);
     }
+    // fp32 and fp64, and the any-shape kernel: the form always (choose_form)
+    if (f.family == kAnyShape || f.family == kWide) return 1e9;
+    if (f.family == kUnknown) return 0.0;                            // (a kernel that this table does not know keeps its products)
+    const RegistryCost& c = kRegistryCost[f.family][p.esz == 1u];
+    if (c.bm == 0u) return 0.0;
+    const auto tiles = [](uint32_t x, uint32_t b, bool whole) { return whole && x > b ? x / b : cdiv(x, b); };
+    const double rounds = (double)cdiv64((uint64_t)tiles(p.s.m, c.bm, f.whole_m) * tiles(p.s.n, c.bn, f.whole_n) * p.batch * ks, p.cus);
+    const double elems = (double)p.s.m * p.s.n * p.batch * 1e-6, mb = p.batch * 1e-6 * p.esz * p.s.k;
+    return c.t0 + rounds * (cdiv(p.steps, ks) * c.step + c.round) + elems * (c.c + c.crange * ks) + c.range * ks +
+           mb * (c.mb * ((double)p.s.m + p.s.n) + c.copy * ((ld.pack_a.on ? (double)p.s.m : 0.0) + (ld.pack_b.on ? (double)p.s.n : 0.0)));
 }
 
 }  // namespace
@@ -148,7 +171,8 @@ const char* form_name(uint32_t index) {
 }
 
 bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t compute_units, FormPlan* out) {
-    const Family fam = families()[registry];
+    const FamilyOf& of = families()[registry];
+    const Family fam = of.family;
     if (compute_units == 0u) return false;
     Problem p;
     p.s = dims_of(d);
@@ -171,14 +195,15 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     p.rows_a = rows16(d.gemm.a.ptr, lda, d.gemm.stride_a);
     p.rows_b = rows16(d.gemm.b.ptr, ldb, d.gemm.stride_b);
     const double c_bytes = fam == kWide ? p.esz : d.out_type == MAIZE_OUT_F32 ? 4.0 : 2.0;
-    p.bytes = p.batch * (p.esz * ((double)p.s.m + p.s.n) * p.s.k + c_bytes * p.s.m * p.s.n * (d.beta != 0.0f ? 2.0 : 1.0));
+    p.ab_bytes = (double)p.batch * p.esz * ((double)p.s.m + p.s.n) * p.s.k;
+    p.bytes = p.ab_bytes + p.batch * c_bytes * p.s.m * p.s.n * (d.beta != 0.0f ? 2.0 : 1.0);
 
     LaunchDims ld;
     std::memset(&ld, 0, sizeof ld);
     if (!kernel_at(registry).plan(d, compute_units, &ld)) return false;       // (what the registry's kernel refuses stays refused)
-    // fp32 and fp64: the form always.  Of 1977 drawn products the registry's 128 x 128 tiles through registers were ahead of the
-    // best tile on four, by 3 % at most, and 4.3 times as long on average.
-    const double rival = fam == kAnyShape || fam == kWide ? 1e9 : registry_cost(fam, p, ld.ksplit);
+    // fp32 and fp64: the form always.  The registry's 128 x 128 tiles through registers take 4.3 (fp64 5.7) times as long on the
+    // average of 2000 drawn products; they are more than 3 % ahead on 41, at most 24 %, most of them a short K with many tiles.
+    const double rival = registry_cost(of, p, ld);
 
     // The any-shape kernel multiplies 8-bit operands widened to bf16: its form does too.  Everywhere else the other tiles.
     const bool widened = bits8 && fam == kAnyShape;
@@ -207,17 +232,22 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
             if (cost < best * (big ? 0.92 : 1.0)) { best = cost; tile = t; ranges = ks; }
         }
     }
-    // The form has to win 10 % by the model: of 590 products the choice is then 1.4 % behind the best of all candidates on
-    // average, and six are slower than with the registry kernel alone, by 3 to 19 % (none allowed: 1.86x on average, all: 1.855x).
-    if (best >= 0.9 * rival) return false;
+    const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][tile] : kTileCost[tile];
+    const uint64_t tiles = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch, items = tiles * ranges;
+    // The form has to win by the model; by 8 % against 128-row tiles and K ranges above 64 rows, by 10 % against the few-row kernels
+    // (the shares that left the sum of all times least).  Of 4000 drawn products 3352 then run a form, in 0.47 of the registry
+    // kernel's time on average; 42 of them are more than 3 % slower on it, 20 more than 10 %, at most 29 % (with one share of 0.9, and
+    // without wait_factor: 68 of all 4000, 41 and 54 %).
+    const bool few_rows = fam == kSkinnyNN || fam == kSkinnyNT;
+    const bool close = fam == kH128 || fam == kH128Gen || fam == kH128R3 || fam == kH128R3Gen || fam == kH128Split || fam == kMT256Split;
+    const double share = few_rows ? 0.9 : close && p.s.m > 64u ? 0.92 : 1.0;
+    if (best >= 1e9 || (rival < 1e9 && tile_cost(c, p, tiles, ranges, few_rows ? 1.0 : wait_factor(c, p)) >= share * rival)) return false;
     // A product that the launcher would cut was compared with its uncut kernel only: it stays cut (4453 x 3712 x 2432 71 us against
     // 79 on the form, 816 x 18448 x 11456 320 against 465, E4M3 1387 x 11200 x 15040 214 against 316).
-    if (fam == kMT256 && cdiv64((uint64_t)cdiv(p.s.m, 256) * cdiv(p.s.n, 256), compute_units) > 1u) {
+    if ((fam == kMT256 || fam == kMT256Gen) && cdiv64((uint64_t)cdiv(p.s.m, 256) * cdiv(p.s.n, 256), compute_units) > 1u) {
         const TailSplit cut = tail_split(d, compute_units);
         if (cut.rows || cut.cols) return false;
     }
-    const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][tile] : kTileCost[tile];
-    const uint64_t items = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch * ranges;
     out->kernel = (d.in_type * 2u + (p.s.nt ? 1u : 0u)) * kTiles + tile;
     out->grid = (uint32_t)items;
     out->ksplit = ranges;
