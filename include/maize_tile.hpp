@@ -265,9 +265,16 @@ class LoadedGemm {
         uint32_t cus = 256;
         maize_device_info_t info;
         if (maize_hip_device_info(ctx.handle(), &info) == MAIZE_OK) cus = info.compute_units;
+        const bool described = op.family == Family::MT256 && op.pipe;
         if (op.family == Family::WAVE32) forced_ = "maize_gemm_bf16_wave32";
-        else if (op.family == Family::MT256 && op.pipe) forced_ = described_kernel(x_, op.nt, op.panel_rows, op.pipe, cus, op.panel_cols);
+        else if (described) forced_ = described_kernel(x_, op.nt, op.panel_rows, op.pipe, cus, op.panel_cols);
+        maize_gemm_plan_t form;
+        check(maize_hip_gemm_ex_form(&x_, cus, &form));
         check(maize_hip_gemm_ex_plan(&x_, forced(), cus, &plan_));
+        if (form.kernel[0] && !forced()) {
+            if (described) forced_ = plan_.kernel;    // of the described family; unnamed, the form would run
+            else plan_ = form;
+        }
     }
     std::string kernel_name() const { return plan_.kernel; }
     const maize_gemm_plan_t& plan() const { return plan_; }

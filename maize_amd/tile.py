@@ -18,7 +18,7 @@ launch ``maize_hip_gemm_bf16[_ex]`` makes for the same operands.
 from dataclasses import dataclass
 
 from . import _ffi
-from .api import Gfx, Matrix, gemm_ex_desc, gemm_plan
+from .api import Gfx, Matrix, gemm_ex_desc, gemm_form, gemm_plan
 
 # ---- tile types and shared-memory tiles ---------------------------------------------------------
 
@@ -404,8 +404,11 @@ class PreLoadGemm:
         desc = gemm_ex_desc(a, b, c, layout=_ffi.LAYOUT_NT if op["nt"] else _ffi.LAYOUT_NN, out_type=op["out_type"], alpha=op["alpha"],
                             beta=op["beta"], in_type=op["mma"].in_type)
         forced = "maize_gemm_bf16_wave32" if op["mma"].family == "wave32" else None
+        cus = ctx.info()["compute_units"]
         if op["mma"].family == "mt256":
-            forced = described_kernel(desc, op["mma"], op["nt"], op["panel_rows"], op["pipe"], ctx.info()["compute_units"], op["panel_cols"])
+            forced = described_kernel(desc, op["mma"], op["nt"], op["panel_rows"], op["pipe"], cus, op["panel_cols"])
+            if forced is None and gemm_form(desc, compute_units=cus):
+                forced = gemm_plan(desc, compute_units=cus)["kernel"]     # of the described family; unnamed, the form would run
         return LoadedGemm(ctx, desc, forced, op["mma"])
 
 
@@ -414,7 +417,8 @@ class LoadedGemm:
 
     def __init__(self, ctx, desc, forced, mma):
         self.ctx, self.desc, self.forced, self.mma = ctx, desc, forced, mma
-        self.plan = gemm_plan(desc, kernel=forced, compute_units=ctx.info()["compute_units"])
+        cus = ctx.info()["compute_units"]
+        self.plan = (None if forced else gemm_form(desc, compute_units=cus)) or gemm_plan(desc, kernel=forced, compute_units=cus)
 
     @property
     def kernel_name(self):

@@ -244,3 +244,39 @@ int main() {
     subprocess.run(["g++", "-O1", "-std=c++17", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-o", str(exe), str(src), os.path.join(CSRC, "dispatch.cpp")], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
+
+
+def test_a_kernel_described_in_cpp_is_not_replaced_by_a_form(tmp_path):
+    """include/maize_tile.hpp: a described mainloop launches its kernel also where the launcher, left the choice, would run a
+    form (512 x 1024 x 1024)."""
+    src = tmp_path / "described.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include "maize_tile.hpp"
+using namespace maize;
+extern "C" const char* fake_log();
+extern "C" void fake_memory(size_t);
+int main() {
+    fake_memory((size_t)1 << 40);
+    Ctx ctx(0);
+    const Matrix a = Matrix::make((BF16*)0x100000000, 512, 1024), b = Matrix::make((BF16*)0x200000000, 1024, 1024), c = Matrix::make((BF16*)0x300000000, 512, 1024);
+    TracedKernel k = new_hip_kernel();
+    k.with_launch_bounds_2d({256, 1});
+    auto ring = k.alloc_aligned_shared<TilePair<Tile<BF16_128x64>, Tile<BF16_64x128>>, 4>(1024);
+    const Wave wave{k.cx()};
+    collective_aligned_row_panel_iter<128>(a, BlockX{k.cx()}).first.for_every_value([&](const RowPanel<128>& ap) {
+        collective_aligned_col_panel_iter<128>(b, BlockY{k.cx()}).first.for_every_value([&](const ColPanel<128>& bp) {
+            gemm_smem_multibuffer(Gfx950MfmaBf16F32_16x16x32{}, KTile<64>{}, ap, bp, ring, wave, 16).store(c);
+        });
+    });
+    LoadedGemm g = k.finalize().compile(Gfx::Gfx950, ctx);
+    g.launch();
+    std::printf("%s\n%s", g.kernel_name().c_str(), fake_log());
+}
+''')
+    exe = tmp_path / "described"
+    cpp = [os.path.join(CSRC, f) for f in ("shim.cpp", "dispatch.cpp", "forms.cpp")] + [os.path.join(ROOT, "tests", "cpu", "fake_hip.cpp")]
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-o", str(exe), str(src)] + cpp, check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+    assert mz.gemm_form(product(512, 1024, 1024)) is not None
+    assert out.splitlines()[0] == "maize_gemm_bf16_t128_nn" and any(l.startswith("launch") and "maize_gemm_bf16_t128_nn" in l for l in out.splitlines()), out

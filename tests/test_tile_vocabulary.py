@@ -167,6 +167,25 @@ def test_the_description_chooses_the_panel_height_and_the_ring_depth():
         k.finalize().compile(mz.Gfx.Gfx950, cus)
 
 
+@pytest.mark.parametrize("shape,kw,kernel", [
+    ((512, 1024, 1024, False), dict(depth=4, a_panel=128, panel=128, tiles=(T.BF16_128x64, T.BF16_64x128)), "maize_gemm_bf16_t128_nn"),
+    ((520, 776, 328, False), dict(depth=2, a_panel=128, tiles=(T.BF16_128x64, T.BF16_64x256)), "maize_gemm_bf16_mt256_nn_h128_gen"),
+    ((64, 64, 1999, False), dict(), "maize_gemm_bf16_mt256_nn_packed"),
+    ((16, 4096, 4096, True), dict(nt=True, tiles=(T.BF16_256x64, T.BF16_256x64)), "maize_gemm_bf16_skinny_nt")], ids=lambda x: x if isinstance(x, str) else None)
+def test_a_described_kernel_is_not_replaced_by_a_form(shape, kw, kernel):
+    """Products that the launcher runs on a form of its own when no kernel is named: the description names one."""
+    a, b, c = matrices(*shape)
+    loaded = describe(a, b, c, **kw)[0].finalize().compile(mz.Gfx.Gfx950, FakeCtx())
+    assert mz.gemm_form(loaded.desc) is not None
+    assert loaded.forced == loaded.kernel_name == kernel and loaded.plan == mz.gemm_plan(loaded.desc, kernel=kernel)
+
+
+def test_a_description_without_panels_tells_the_form_that_runs():
+    """fp32 operands: the description fixes the instruction only, the choice is the launcher's."""
+    loaded = describe(*matrices(1000, 1000, 1000), mma=T.Gfx950MfmaF32F32_16x16x4, ktile=32, ring=False)[0].finalize().compile(mz.Gfx.Gfx950, FakeCtx())
+    assert loaded.forced is None and loaded.plan == mz.gemm_form(loaded.desc) and loaded.kernel_name.startswith("maize_tile_f32_nn_")
+
+
 def test_trace_errors():
     a, b, c = matrices(512, 512, 512)
     with pytest.raises(ValueError, match="inner dimensions differ"):
