@@ -148,29 +148,42 @@ def test_full_precision_forms_at_their_edges(ctx, oracle, forms, ty, tile, layou
         check(bm + 3, bn + 5, k, ks=ks)
 
 
-def test_captured_products_keep_no_address_of_a_workspace_that_may_be_freed(ctx):
-    """A product whose form splits K, captured where the stream's workspace is large enough already; a larger product then
-    replaces that workspace.  Every replay equals the product of the captured inputs."""
+@pytest.mark.parametrize("warm", [True, False], ids=["run-before", "first-call"])
+def test_a_captured_form_in_k_ranges_equals_the_eager_one(ctx, warm):
+    """A product whose form splits K, captured where the stream's workspace holds it and where the stream has none yet; between
+    the replays a larger product runs on the stream and replaces the workspace.  Every replay has the bits of the eager call."""
     hip = _ffi.lib()                                          # (the HIP runtime's own functions, through the library that links it)
 
     def call(f, *args):
         assert getattr(hip, f)(*args) == 0, f
 
-    m, n, k = 64, 64, 777
-    rng = np.random.default_rng(5)
-    a, b = (rng.integers(-3, 4, s).astype(np.float32) for s in ((m, k), (k, n)))          # (integers: any order of the sums, the same bits)
-    bits = lambda x: (x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16).ravel()
-    la, lb = np.ones((512, 8192)), np.ones((8192, 1024))
-    da, db, dla, dlb = (ctx.upload(bits(x)) for x in (a, b, la, lb))
+    cus = ctx.info()["compute_units"]
+    m, n, k = 64, 64, 1999
+    a, b = mz.gen.uniform_bf16(m * k, 5), mz.gen.uniform_bf16(k * n, 6)
+    one = np.full(512 * 8192, 0x3F80, np.uint16)
+    da, db, dla, dlb = ctx.upload(a), ctx.upload(b), ctx.upload(one), ctx.upload(np.concatenate([one, one]))
     dc, dlc = ctx.malloc(m * n * 4), ctx.malloc(512 * 1024 * 4)
-    desc = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), in_type=mz.IN_BF16, out_type=mz.OUT_F32)
-    larger = mz.gemm_ex_desc(mz.Matrix(dla, 512, 8192), mz.Matrix(dlb, 8192, 1024), mz.Matrix(dlc, 512, 1024), in_type=mz.IN_BF16, out_type=mz.OUT_F32)
+    desc = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), out_type=mz.OUT_F32)
+    larger = mz.gemm_ex_desc(mz.Matrix(dla, 512, 8192), mz.Matrix(dlb, 8192, 1024), mz.Matrix(dlc, 512, 1024), out_type=mz.OUT_F32)
+    form, grows = mz.gemm_form(desc, cus), mz.gemm_form(larger, cus)
+    assert form["ksplit"] > 1 and 2 * form["workspace_bytes"] < grows["workspace_bytes"], (form, grows)
+    other = ctx.stream()
+    ctx.gemm_bf16(desc, other)
+    ctx.sync(other)
+    want = dc.download(np.float32)
+    fa, fb = ((x.astype(np.uint32) << 16).view(np.float32).astype(np.float64) for x in (a, b))
+    fa, fb = fa.reshape(m, k), fb.reshape(k, n)
+    assert (np.abs(want.reshape(m, n) - fa @ fb) <= (k / 16.0 + 4.0) * 2.0 ** -24 * (np.abs(fa) @ np.abs(fb))).all()
     s, graph, run = ctx.stream(), C.c_void_p(), C.c_void_p()
-    ctx.gemm_bf16(desc, s)
-    ctx.sync(s)
+    if warm:
+        ctx.gemm_bf16(desc, s)
+        ctx.sync(s)
     call("hipStreamBeginCapture", s, 1)
     ctx.gemm_bf16(desc, s)
     call("hipStreamEndCapture", s, C.byref(graph))
+    nodes = C.c_size_t()
+    call("hipGraphGetNodes", graph, None, C.byref(nodes))
+    assert nodes.value == 1
     call("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
     for i in range(3):
         dc.fill(0)
@@ -178,12 +191,13 @@ def test_captured_products_keep_no_address_of_a_workspace_that_may_be_freed(ctx)
         print(f"replay {i}", flush=True)
         call("hipGraphLaunch", run, s)
         ctx.sync(s)
-        assert np.array_equal(dc.download(np.float32).reshape(m, n), a @ b)
+        assert np.array_equal(dc.download(np.float32), want)
         ctx.gemm_bf16(larger, s)
         ctx.sync(s)
         assert (dlc.download(np.float32) == 8192.0).all()
     call("hipGraphExecDestroy", run)
     call("hipGraphDestroy", graph)
     ctx.stream_destroy(s)
+    ctx.stream_destroy(other)
     for x in (da, db, dla, dlb, dc, dlc):
         x.free()
