@@ -11,6 +11,15 @@ def f32_of(bits):
     return (np.asarray(bits, dtype=np.uint16).astype(np.uint32) << 16).view(np.float32)
 
 
+def kernels_of(ctx, desc, kernel=None):
+    """What a test of `desc` launches: the kernel that it names; or, where it names none, the launcher's choice (None) and,
+    where that is one of the launcher's own forms, by name the registry kernel that the plan reports as well."""
+    cus = ctx.info()["compute_units"]
+    if kernel is not None or mz.gemm_form(desc, compute_units=cus) is None:
+        return [kernel]
+    return [None, mz.gemm_plan(desc, compute_units=cus)["kernel"]]
+
+
 def run_gemm(ctx, a, b, m, n, k, layout=mz.LAYOUT_NN, batch=1, stride_a=None, stride_b=None, stride_c=None,
              kernel=None, stream=None):
     """C = A.B on the device through maize_hip_gemm_bf16[_with]; returns C as uint16 of

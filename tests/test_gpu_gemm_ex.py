@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import maize_amd as mz
+from tests.gpu_util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -24,7 +25,8 @@ def _say(msg):
 def run_ex(ctx, oracle, m, n, k, layout=mz.LAYOUT_NN, lda=None, ldb=None, ldc=None, alpha=1.0, beta=0.0, out_f32=False,
            kernel=None, seed=1, c_nan=False, label="", half=False):
     """One launch on padded views whose padding (and C's) holds canaries; checks the result against the
-    oracle and that nothing outside the M x N view of C changed.  Returns the kernel the dispatcher took."""
+    oracle and that nothing outside the M x N view of C changed.  Returns the kernel the dispatcher took: where the launcher
+    runs one of its forms in its place, both are launched and checked."""
     brows, bcols = (k, n) if layout == mz.LAYOUT_NN else (n, k)
     lda = k if lda is None else lda
     ldb = bcols if ldb is None else ldb
@@ -53,24 +55,27 @@ def run_ex(ctx, oracle, m, n, k, layout=mz.LAYOUT_NN, lda=None, ldb=None, ldc=No
                             in_type=mz.IN_F16 if half else mz.IN_BF16)
         took = mz.gemm_plan(x, kernel=kernel, compute_units=ctx.info()["compute_units"])["kernel"]
         _say(f"{label} M={m} N={n} K={k} ld=({lda},{ldb},{ldc}) alpha={alpha} beta={beta} f32={out_f32} -> {took}")
-        ctx.gemm_bf16(x, kernel=kernel)
-        ctx.sync()
-        got = dc.download(cdt)
+        results = []
+        for named in kernels_of(ctx, x, kernel):
+            dc.write(c0)
+            ctx.gemm_bf16(x, kernel=named)
+            ctx.sync()
+            results.append(dc.download(cdt).reshape(m, ldc))
     finally:
         da.free(); db.free(); dc.free()
-    gv = got.reshape(m, ldc)
     ov = c0.reshape(m, ldc)
-    # the padding of C's rows is untouched (bit for bit)
-    assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
     ref, val, scale = oracle.ref_gemm_ex(a, b, m, n, k, layout=layout, lda=lda, ldb=ldb, alpha=alpha, beta=beta,
                                          c_old=None if beta == 0.0 else ov[:, :n].copy(), out_f32=out_f32,
                                          elem=oracle.F16 if half else oracle.BF16)
-    g = gv[:, :n]
-    if out_f32:
-        check_f32_c(oracle, g, val, scale, a, b, m, n, k, layout, lda, ldb, alpha, beta, None if beta == 0.0 else ov[:, :n], half, label)
-    else:
-        s = oracle.compare(g, ref, val, scale, k, elem=oracle.F16 if half else oracle.BF16)
-        oracle.assert_parity(s, label)
+    for gv in results:
+        # the padding of C's rows is untouched (bit for bit)
+        assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+        g = gv[:, :n]
+        if out_f32:
+            check_f32_c(oracle, g, val, scale, a, b, m, n, k, layout, lda, ldb, alpha, beta, None if beta == 0.0 else ov[:, :n], half, label)
+        else:
+            s = oracle.compare(g, ref, val, scale, k, elem=oracle.F16 if half else oracle.BF16)
+            oracle.assert_parity(s, label)
     return took
 
 
@@ -137,11 +142,13 @@ def test_macro_tile_view_of_a_larger_matrix_matches_the_compact_run(ctx, oracle)
         dc = ctx.malloc(m * (lc or n) * 2)
         dc.fill(0)
         x = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), lda=la, ldb=lb, ldc=lc)
-        ctx.gemm_bf16(x)
-        ctx.sync()
-        outs.append(dc.download(np.uint16).reshape(m, lc or n)[:, :n].copy())
+        for kernel in kernels_of(ctx, x):
+            dc.fill(0)
+            ctx.gemm_bf16(x, kernel=kernel)
+            ctx.sync()
+            outs.append(dc.download(np.uint16).reshape(m, lc or n)[:, :n].copy())
         da.free(); db.free(); dc.free()
-    assert np.array_equal(outs[0], outs[1])
+    assert len(outs) in (2, 4) and all(np.array_equal(x, y) for x, y in zip(outs, outs[len(outs) // 2:]))
 
 
 @pytest.mark.parametrize("m", [1, 7, 16])
@@ -180,8 +187,8 @@ def test_macro_tile_general_epilogue(ctx, oracle, layout, shape, lds):
 
 
 def test_general_epilogue_with_several_tiles_per_workgroup_and_batches(ctx, oracle):
-    """A batched fp32 product with beta, through the dispatcher (which takes 128-row tiles for it: 18 of them) and
-    through the 256-row general kernel by name."""
+    """A batched fp32 product with beta, left to the launcher, through the dispatcher's kernel (128 x 128 tiles) and through the
+    128- and 256-row general kernels by name."""
     m, n, k, batch = 256, 384, 128, 3
     a = mz.gen.uniform_bf16(batch * m * k, 21)
     b = mz.gen.uniform_bf16(batch * k * n, 22)
@@ -191,7 +198,7 @@ def test_general_epilogue_with_several_tiles_per_workgroup_and_batches(ctx, orac
         x = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), batch=batch, stride_a=m * k,
                             stride_b=k * n, stride_c=m * n, out_type=mz.OUT_F32, alpha=0.75, beta=1.5)
         assert mz.gemm_plan(x)["kernel"] == "maize_gemm_bf16_t128_nn"
-        for kernel in (None, "maize_gemm_bf16_mt256_nn_h128_gen", "maize_gemm_bf16_mt256_nn_gen"):
+        for kernel in (None, "maize_gemm_bf16_t128_nn", "maize_gemm_bf16_mt256_nn_h128_gen", "maize_gemm_bf16_mt256_nn_gen"):
             dc.write(c0)
             ctx.gemm_bf16(x, kernel=kernel)
             ctx.sync()
@@ -299,16 +306,21 @@ def test_half_operands_out_f16_is_out_same(ctx, oracle):
             dc = ctx.upload(np.zeros(m * n, np.uint16))
             x = mz.gemm_ex_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n), mz.Matrix(dc, m, n), out_type=ot, in_type=mz.IN_F16)
             took = mz.gemm_plan(x, compute_units=ctx.info()["compute_units"])["kernel"]
-            ctx.gemm_bf16(x)
-            ctx.sync()
-            out[name] = (took, dc.download(np.uint16))
+            results = []
+            for kernel in kernels_of(ctx, x):
+                ctx.gemm_bf16(x, kernel=kernel)
+                ctx.sync()
+                results.append(dc.download(np.uint16))
+                dc.fill(0)
+            out[name] = (took, results)
             dc.free()
     finally:
         da.free(); db.free()
-    assert out["same"][0] == out["f16"][0]
-    assert np.array_equal(out["same"][1], out["f16"][1])
+    assert out["same"][0] == out["f16"][0] and len(out["same"][1]) == len(out["f16"][1])
     ref, val, scale = oracle.ref_gemm_ex(a, b, m, n, k, elem=oracle.F16)
-    oracle.assert_parity(oracle.compare(out["f16"][1], ref, val, scale, k, elem=oracle.F16), "half C")
+    for same, half in zip(out["same"][1], out["f16"][1]):
+        assert np.array_equal(same, half)
+        oracle.assert_parity(oracle.compare(half, ref, val, scale, k, elem=oracle.F16), "half C")
 
 
 @pytest.mark.parametrize("m", [3, 16])
@@ -426,23 +438,28 @@ def run_packed(ctx, oracle, m, n, k, layout, kernel, lda=None, ldb=None, ldc=Non
                             in_type=mz.IN_F16 if half else mz.IN_BF16)
         took = mz.gemm_plan(x, kernel=kernel, compute_units=ctx.info()["compute_units"])["kernel"]
         _say(f"{label} M={m} N={n} K={k} ld=({lda},{ldb},{ldc}) off=({a_off},{b_off},{c_off}) alpha={alpha} beta={beta} f32={out_f32} half={half} -> {took}")
-        ctx.gemm_bf16(x, kernel=kernel)
-        ctx.sync()
-        got = dc.download(np.float32 if out_f32 else np.uint16)
+        results = []
+        for named in kernels_of(ctx, x, kernel):
+            dc.write(c0)
+            ctx.gemm_bf16(x, kernel=named)
+            ctx.sync()
+            results.append(dc.download(np.float32 if out_f32 else np.uint16))
     finally:
         da.free(); db.free(); dc.free()
-    assert np.array_equal(got[:c_off].view(np.uint8), c0[:c_off].view(np.uint8)), f"{label}: wrote before C"
-    gv, ov = got[c_off:].reshape(m, ldc), c0[c_off:].reshape(m, ldc)
-    assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+    ov = c0[c_off:].reshape(m, ldc)
     elem = oracle.F16 if half else oracle.BF16
     ref, val, scale = oracle.ref_gemm_ex(a[a_off:], b[b_off:], m, n, k, layout=layout, lda=lda, ldb=ldb, alpha=alpha, beta=beta,
                                          c_old=None if beta == 0.0 else ov[:, :n].copy(), out_f32=out_f32, elem=elem)
-    g = gv[:, :n]
-    if out_f32:
-        check_f32_c(oracle, g, val, scale, a[a_off:], b[b_off:], m, n, k, layout, lda, ldb, alpha, beta, None if beta == 0.0 else ov[:, :n], half, label)
-    else:
-        s = oracle.compare(g, ref, val, scale, k, elem=elem)
-        oracle.assert_parity(s, label)
+    for got in results:
+        assert np.array_equal(got[:c_off].view(np.uint8), c0[:c_off].view(np.uint8)), f"{label}: wrote before C"
+        gv = got[c_off:].reshape(m, ldc)
+        assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+        g = gv[:, :n]
+        if out_f32:
+            check_f32_c(oracle, g, val, scale, a[a_off:], b[b_off:], m, n, k, layout, lda, ldb, alpha, beta, None if beta == 0.0 else ov[:, :n], half, label)
+        else:
+            s = oracle.compare(g, ref, val, scale, k, elem=elem)
+            oracle.assert_parity(s, label)
     return took
 
 
@@ -492,15 +509,19 @@ def test_packed_path_is_what_odd_large_shapes_get(ctx, oracle):
         d = mz.gemm_desc(mz.Matrix(da, m, k), mz.Matrix(db, brows, bcols), mz.Matrix(dc, m, n), layout=layout)
         took = ctx.gemm_select(d)
         assert took.endswith(want), took
-        _say(f"odd large shape {m}x{n}x{k} -> {took}")
-        ctx.gemm_bf16(d)
-        ctx.sync()
-        got = dc.download(np.uint16).reshape(m, n)
-        da.free(); db.free(); dc.free()
         rows = sample_rows(m, count=24)
         ref, f64, ab = oracle.ref_gemm_rows(a, b, m, n, k, rows, layout=layout)
-        s = oracle.compare(got[rows], ref, f64, ab, k)
-        oracle.assert_parity(s, f"odd large shape {m}x{n}x{k} {took}")
+        kernels = kernels_of(ctx, d)
+        assert kernels[-1] == took                    # (the launcher runs a form in its place: both are checked)
+        for kernel in kernels:
+            _say(f"odd large shape {m}x{n}x{k} -> {kernel or 'a form'}")
+            dc.fill(0xFF)
+            ctx.gemm_bf16(d, kernel=kernel)
+            ctx.sync()
+            got = dc.download(np.uint16).reshape(m, n)
+            s = oracle.compare(got[rows], ref, f64, ab, k)
+            oracle.assert_parity(s, f"odd large shape {m}x{n}x{k} {kernel}")
+        da.free(); db.free(); dc.free()
 
 
 def test_packed_batched(ctx, oracle):

@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 import maize_amd as mz
+from tests.gpu_util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -37,7 +38,9 @@ def ab_of(elem):
 
 
 def launch(ctx, a, b, c0, m, n, k, layout, fmt, lda, ldb, ldc, alpha=1.0, beta=0.0, out_f32=False, kernel=None, batch=1,
-           strides=(0, 0, 0), out_f16=False):
+           strides=(0, 0, 0), out_f16=False, forms_too=False):
+    """(C, the kernel of the plan).  forms_too: a list of C's instead -- without a kernel named, of the launcher's choice and,
+    where that is one of its forms, of the plan's kernel by name."""
     brows, bcols = (k, n) if layout == mz.LAYOUT_NN else (n, k)
     da, db, dc = ctx.upload(a), ctx.upload(b), ctx.upload(c0)
     try:
@@ -46,12 +49,15 @@ def launch(ctx, a, b, c0, m, n, k, layout, fmt, lda, ldb, ldc, alpha=1.0, beta=0
                             out_type=mz.OUT_F32 if out_f32 else mz.OUT_F16 if out_f16 else mz.OUT_SAME, alpha=alpha, beta=beta, in_type=FMT[fmt][0],
                             batch=batch, stride_a=strides[0], stride_b=strides[1], stride_c=strides[2])
         took = mz.gemm_plan(x, kernel=kernel, compute_units=ctx.info()["compute_units"])["kernel"]
-        ctx.gemm_bf16(x, kernel=kernel)
-        ctx.sync()
-        got = dc.download(np.float32 if out_f32 else np.uint16)
+        results = []
+        for named in kernels_of(ctx, x, kernel) if forms_too else [kernel]:
+            dc.write(c0)
+            ctx.gemm_bf16(x, kernel=named)
+            ctx.sync()
+            results.append(dc.download(np.float32 if out_f32 else np.uint16))
     finally:
         da.free(); db.free(); dc.free()
-    return got, took
+    return results if forms_too else results[0], took
 
 
 def run_f8(ctx, oracle, m, n, k, layout=mz.LAYOUT_NT, fmt="e4m3", lda=None, ldb=None, ldc=None, alpha=1.0, beta=0.0,
@@ -69,25 +75,27 @@ def run_f8(ctx, oracle, m, n, k, layout=mz.LAYOUT_NT, fmt="e4m3", lda=None, ldb=
         c0 = oracle.bf16_bits_from_f64(np.random.default_rng(seed).random(m * ldc) * 2.0 - 1.0, oracle.F16)
     else:
         c0 = mz.gen.uniform_bf16(m * ldc, 300 + seed)
-    got, took = launch(ctx, a, b, c0, m, n, k, layout, fmt, lda, ldb, ldc, alpha, beta, out_f32, kernel, out_f16=out_f16)
+    results, took = launch(ctx, a, b, c0, m, n, k, layout, fmt, lda, ldb, ldc, alpha, beta, out_f32, kernel, out_f16=out_f16, forms_too=True)
     _say(f"{label} {fmt} M={m} N={n} K={k} ld=({lda},{ldb},{ldc}) alpha={alpha} beta={beta} f32={out_f32} f16={out_f16} -> {took}")
-    gv, ov = got.reshape(m, ldc), c0.reshape(m, ldc)
-    assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+    ov = c0.reshape(m, ldc)
     ref, val, scale = oracle.ref_gemm_ex(a, b, m, n, k, layout=layout, lda=lda, ldb=ldb, alpha=alpha, beta=beta,
                                          c_old=None if beta == 0.0 else ov[:, :n].copy(), out_f32=out_f32, elem=elem,
                                          c_elem=oracle.F16 if out_f16 else None)
-    g = gv[:, :n]
-    f8_unit = "wave32" not in took               # every other kernel multiplies with the 8-bit matrix instruction
-    if out_f32:
-        err = np.abs(g.astype(np.float64) - val)
-        tol = ((oracle.floor_coeff_f8(k) + 2.0 ** -23) if f8_unit else (k / 16.0 + 4.0) * 2.0 ** -24) * scale + 1e-45
-        bad = ~(err <= tol)
-        assert not bad.any(), f"{label}: {int(bad.sum())} of {bad.size} fp32 elements out of tolerance, worst {float((err / tol).max()):.2f}x"
-    else:
-        s = oracle.compare(g, ref, val, scale, k, elem=oracle.F16 if out_f16 else oracle.BF16,
-                           coeff=oracle.floor_coeff_f8(k) if f8_unit else None)
-        assert s["n_fail"] == 0, f"{label}: {s}"
-        _say(f"   max_ulp {s['max_ulp']} n_gt1ulp {s['n_gt1ulp']} of {s['n']}")
+    f8_unit = "wave32" not in took               # every other kernel multiplies with the 8-bit matrix instruction (and so does its form)
+    for got in results:
+        gv = got.reshape(m, ldc)
+        assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+        g = gv[:, :n]
+        if out_f32:
+            err = np.abs(g.astype(np.float64) - val)
+            tol = ((oracle.floor_coeff_f8(k) + 2.0 ** -23) if f8_unit else (k / 16.0 + 4.0) * 2.0 ** -24) * scale + 1e-45
+            bad = ~(err <= tol)
+            assert not bad.any(), f"{label}: {int(bad.sum())} of {bad.size} fp32 elements out of tolerance, worst {float((err / tol).max()):.2f}x"
+        else:
+            s = oracle.compare(g, ref, val, scale, k, elem=oracle.F16 if out_f16 else oracle.BF16,
+                               coeff=oracle.floor_coeff_f8(k) if f8_unit else None)
+            assert s["n_fail"] == 0, f"{label}: {s}"
+            _say(f"   max_ulp {s['max_ulp']} n_gt1ulp {s['n_gt1ulp']} of {s['n']}")
     return took
 
 
@@ -484,11 +492,12 @@ def test_split_k_on_8bit_operands(ctx, oracle, fmt):
     m, n, k = 24, 520, 4096
     a = f8_uniform(oracle, m * k, 31, elem)
     b = f8_uniform(oracle, n * k, 32, elem)
-    first, took = launch(ctx, a, b, np.zeros(m * n, np.uint16), m, n, k, mz.LAYOUT_NT, fmt, k, k, n)
-    assert took == half_tiles
-    for _ in range(3):
-        again, _ = launch(ctx, a, b, np.full(m * n, 0x7FC0, np.uint16), m, n, k, mz.LAYOUT_NT, fmt, k, k, n)
-        assert np.array_equal(again, first)
+    for kernel in (None, half_tiles):                             # (the launcher runs a form in its place)
+        first, took = launch(ctx, a, b, np.zeros(m * n, np.uint16), m, n, k, mz.LAYOUT_NT, fmt, k, k, n, kernel=kernel)
+        assert took == half_tiles
+        for _ in range(3):
+            again, _ = launch(ctx, a, b, np.full(m * n, 0x7FC0, np.uint16), m, n, k, mz.LAYOUT_NT, fmt, k, k, n, kernel=kernel)
+            assert np.array_equal(again, first)
     # the bf16 skinny kernel shares the stream's workspace (its ticket counters must still be zero)
     m2, n2, k2 = 16, 1096, 4096
     a2 = mz.gen.normal_bf16(m2 * k2, 3, 1.0)
@@ -497,7 +506,7 @@ def test_split_k_on_8bit_operands(ctx, oracle, fmt):
     try:
         d = mz.gemm_desc(mz.Matrix(da, m2, k2), mz.Matrix(db, k2, n2), mz.Matrix(dc, m2, n2))
         assert mz.gemm_plan(d, compute_units=ctx.info()["compute_units"])["kernel"] == "maize_gemm_bf16_skinny_nn"
-        ctx.gemm_bf16(d)
+        ctx.gemm_bf16(d, kernel="maize_gemm_bf16_skinny_nn")
         ctx.sync()
         got = dc.download(np.uint16)
     finally:
@@ -556,10 +565,11 @@ def test_packed_path_for_8bit_operands(ctx, oracle, fmt):
     sa, sb, sc = m * k + 3, k * n + 5, m * n + 8
     ab_ = f8_uniform(oracle, batch * sa, 61, ab_of(elem)[0])
     bb_ = f8_uniform(oracle, batch * sb, 62, ab_of(elem)[1])
-    dense, took = launch(ctx, ab_, bb_, np.zeros(batch * sc, np.uint16), m, n, k, NN, fmt, k, n, n, batch=batch, strides=(sa, sb, sc))
+    _, took = launch(ctx, ab_, bb_, np.zeros(batch * sc, np.uint16), m, n, k, NN, fmt, k, n, n, batch=batch, strides=(sa, sb, sc))
     assert took == name                                           # the odd strides make A unaligned too
+    dense, _ = launch(ctx, ab_, bb_, np.zeros(batch * sc, np.uint16), m, n, k, NN, fmt, k, n, n, batch=batch, strides=(sa, sb, sc), kernel=name)
     for i in range(batch):
-        single, _ = launch(ctx, ab_[i * sa:i * sa + m * k], bb_[i * sb:i * sb + k * n], np.zeros(m * n, np.uint16), m, n, k, NN, fmt, k, n, n)
+        single, _ = launch(ctx, ab_[i * sa:i * sa + m * k], bb_[i * sb:i * sb + k * n], np.zeros(m * n, np.uint16), m, n, k, NN, fmt, k, n, n, kernel=name)
         assert np.array_equal(single, dense[i * sc:i * sc + m * n]), i
         assert not dense[i * sc + m * n:(i + 1) * sc].any(), "wrote between batch members"
 
@@ -595,13 +605,14 @@ def test_half_c_is_rounded_to_half_not_through_bf16(ctx, oracle):
     a = np.full(m * k, one, dtype=np.uint8)
     b = np.full(n * k, one, dtype=np.uint8)
     c0 = np.zeros(m * n, dtype=np.uint16)
-    got, took = launch(ctx, a, b, c0, m, n, k, mz.LAYOUT_NT, "e4m3", k, k, n, out_f16=True)
+    results, took = launch(ctx, a, b, c0, m, n, k, mz.LAYOUT_NT, "e4m3", k, k, n, out_f16=True, forms_too=True)
     _say(f"all-ones K={k} half C -> {took}")
     want = oracle.bf16_bits_from_f64(np.array([4112.0]), oracle.F16)[0]
     assert float(np.array([want], dtype=np.uint16).view(np.float16)[0]) == 4112.0
-    assert np.all(got == want), f"{took}: {np.unique(got)[:8]} instead of {want:#06x}"
-    got_bf16, _ = launch(ctx, a, b, c0, m, n, k, mz.LAYOUT_NT, "e4m3", k, k, n)
-    assert not np.any(oracle.bf16_bits_to_f64(got_bf16) == 4112.0)          # the bf16 C of the same product cannot hold it
+    for got in results:
+        assert np.all(got == want), f"{took}: {np.unique(got)[:8]} instead of {want:#06x}"
+    for got in launch(ctx, a, b, c0, m, n, k, mz.LAYOUT_NT, "e4m3", k, k, n, forms_too=True)[0]:
+        assert not np.any(oracle.bf16_bits_to_f64(got) == 4112.0)           # the bf16 C of the same product cannot hold it
 
 
 @pytest.mark.parametrize("layout", [mz.LAYOUT_NT, mz.LAYOUT_NN], ids=["nt", "nn"])

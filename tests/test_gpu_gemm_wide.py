@@ -6,12 +6,14 @@ Bar.  Exact data (small integers, powers of two): bit for bit.  Random data: |go
 (K/4 + 4) * u * (|alpha| * sum|a||b| + |beta| * |C_old|), u = 2^-24 (fp32) or 2^-53 (fp64): one rounding
 per four-deep matrix instruction on the accumulation path plus the roundings of the epilogue."""
 import ctypes as C
+import itertools
 import sys
 
 import numpy as np
 import pytest
 
 import maize_amd as mz
+from tests.gpu_util import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -24,8 +26,9 @@ def _say(msg):
 
 def launch(ctx, a, b, c0, m, n, k, ty, layout=mz.LAYOUT_NN, lda=None, ldb=None, ldc=None, alpha=1.0, beta=0.0,
            batch=1, strides=(0, 0, 0), offs=(0, 0, 0), kernel=None, label=""):
-    """Uploads flat arrays, launches, returns (C as downloaded, kernel taken).  offs: element offsets of the views
-    inside their buffers (to take pointers that are only element aligned)."""
+    """Uploads flat arrays and launches; returns (C as downloaded by each launch, the plan).  Without a kernel named: the
+    launcher's choice, and where that is one of its forms, the maize_gemm_*_mt128_* kernel of the plan by name.  offs: element
+    offsets of the views inside their buffers (to take pointers that are only element aligned)."""
     dt, in_type = DT[ty]
     brows, bcols = (k, n) if layout == mz.LAYOUT_NN else (n, k)
     da, db, dc = ctx.upload(a), ctx.upload(b), ctx.upload(c0)
@@ -37,9 +40,13 @@ def launch(ctx, a, b, c0, m, n, k, ty, layout=mz.LAYOUT_NN, lda=None, ldb=None, 
         plan = mz.gemm_plan(x, kernel=kernel, compute_units=ctx.info()["compute_units"])
         _say(f"{label} {ty} M={m} N={n} K={k} batch={batch} ld=({lda},{ldb},{ldc}) offs={offs} alpha={alpha} beta={beta} "
              f"-> {plan['kernel']} grid={plan['grid']} vec={plan['split_first']}")
-        ctx.gemm_bf16(x, kernel=kernel)
-        ctx.sync()
-        return dc.download(dt), plan
+        out = []
+        for named in kernels_of(ctx, x, kernel):
+            dc.write(c0)
+            ctx.gemm_bf16(x, kernel=named)
+            ctx.sync()
+            out.append(dc.download(dt))
+        return out, plan
     finally:
         da.free(); db.free(); dc.free()
 
@@ -55,17 +62,18 @@ def run_wide(ctx, oracle, ty, m, n, k, layout=mz.LAYOUT_NN, pad=(0, 0, 0), alpha
     c0 = (rng.standard_normal(offs[2] + m * ldc) * 2).astype(dt)
     if c_nan:
         c0[:] = np.nan
-    got, plan = launch(ctx, a, b, c0, m, n, k, ty, layout, lda if pad[0] else None, ldb if pad[1] else None,
-                       ldc if pad[2] else None, alpha, beta, offs=offs, label=label)
+    results, plan = launch(ctx, a, b, c0, m, n, k, ty, layout, lda if pad[0] else None, ldb if pad[1] else None,
+                           ldc if pad[2] else None, alpha, beta, offs=offs, label=label)
     if want_vec is not None:
         assert plan["split_first"] == want_vec, f"{label}: 128-bit access flags {plan['split_first']}, expected {want_vec}"
-    gv, ov = got[offs[2]:].reshape(m, ldc), c0[offs[2]:].reshape(m, ldc)
-    assert np.array_equal(got[:offs[2]].view(np.uint8), c0[:offs[2]].view(np.uint8)), f"{label}: wrote in front of C"
-    assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
     hi, lo, ab = oracle.ref_gemm_wide(a[offs[0]:], b[offs[1]:], m, n, k, layout=layout, lda=lda, ldb=ldb)
-    worst = oracle.check_wide(gv[:, :n], hi, lo, ab, k, alpha, beta, None if beta == 0.0 else ov[:, :n])
-    _say(f"{label}: worst error / bound = {worst:.3f}")
-    assert worst <= 1.0, f"{label}: error {worst:.2f}x the bound"
+    for got in results:
+        gv, ov = got[offs[2]:].reshape(m, ldc), c0[offs[2]:].reshape(m, ldc)
+        assert np.array_equal(got[:offs[2]].view(np.uint8), c0[:offs[2]].view(np.uint8)), f"{label}: wrote in front of C"
+        assert np.array_equal(gv[:, n:].view(np.uint8), ov[:, n:].view(np.uint8)), f"{label}: wrote into C's row padding"
+        worst = oracle.check_wide(gv[:, :n], hi, lo, ab, k, alpha, beta, None if beta == 0.0 else ov[:, :n])
+        _say(f"{label}: worst error / bound = {worst:.3f}")
+        assert worst <= 1.0, f"{label}: error {worst:.2f}x the bound"
     return plan
 
 
@@ -116,8 +124,9 @@ def test_small_integers_are_exact(ctx, ty, layout):
     A = rng.integers(-8, 9, (m, k)).astype(dt)
     B = rng.integers(-8, 9, (k, n)).astype(dt)
     b = B if layout == mz.LAYOUT_NN else B.T.copy()
-    got, _ = launch(ctx, A.ravel(), b.ravel(), np.zeros(m * n, dt), m, n, k, ty, layout, label="integers")
-    assert np.array_equal(got.reshape(m, n), (A.astype(np.int64) @ B.astype(np.int64)).astype(dt))
+    results, _ = launch(ctx, A.ravel(), b.ravel(), np.zeros(m * n, dt), m, n, k, ty, layout, label="integers")
+    for got in results:
+        assert np.array_equal(got.reshape(m, n), (A.astype(np.int64) @ B.astype(np.int64)).astype(dt))
 
 
 @pytest.mark.parametrize("ty", ["f32", "f64"])
@@ -128,10 +137,12 @@ def test_identity_and_permutation(ctx, ty):
     X = (rng.random((n, n)) * 2 - 1).astype(dt)
     perm = rng.permutation(n)
     P = np.eye(n, dtype=dt)[perm]
-    got, _ = launch(ctx, P.ravel(), X.ravel(), np.zeros(n * n, dt), n, n, n, ty, label="permutation")
-    assert np.array_equal(got.reshape(n, n), X[perm])          # rows of X, moved: exact
-    got, _ = launch(ctx, X.ravel(), np.eye(n, dtype=dt).ravel(), np.zeros(n * n, dt), n, n, n, ty, mz.LAYOUT_NT, label="identity")
-    assert np.array_equal(got.reshape(n, n), X)
+    results, _ = launch(ctx, P.ravel(), X.ravel(), np.zeros(n * n, dt), n, n, n, ty, label="permutation")
+    for got in results:
+        assert np.array_equal(got.reshape(n, n), X[perm])      # rows of X, moved: exact
+    results, _ = launch(ctx, X.ravel(), np.eye(n, dtype=dt).ravel(), np.zeros(n * n, dt), n, n, n, ty, mz.LAYOUT_NT, label="identity")
+    for got in results:
+        assert np.array_equal(got.reshape(n, n), X)
 
 
 @pytest.mark.parametrize("ty", ["f32", "f64"])
@@ -142,9 +153,9 @@ def test_what_fp64_keeps_and_fp32_drops(ctx, ty):
     x = dt(1.0) + dt(2.0 ** -30)
     A = np.zeros((16, 4), dt); A[:, 0] = x
     B = np.zeros((4, 16), dt); B[0, :] = x
-    got, _ = launch(ctx, A.ravel(), B.ravel(), np.zeros(256, dt), 16, 16, 4, ty, label="precision")
+    results, _ = launch(ctx, A.ravel(), B.ravel(), np.zeros(256, dt), 16, 16, 4, ty, label="precision")
     want = dt(1.0) if ty == "f32" else np.float64(1.0) + 2.0 ** -29          # 2^-60 is below fp64's last place
-    assert np.all(got == want)
+    assert all(np.all(got == want) for got in results)
 
 
 # ---- random data, every access path -----------------------------------------------------------------------
@@ -193,8 +204,8 @@ def test_batched(ctx, oracle, ty):
     a = (rng.random(batch * sa) * 2 - 1).astype(dt)
     b = (rng.random(batch * sb) * 2 - 1).astype(dt)
     c0 = rng.standard_normal(batch * sc).astype(dt)
-    got, _ = launch(ctx, a, b, c0, m, n, k, ty, batch=batch, strides=(sa, sb, sc), label="batched")
-    for z in range(batch):
+    results, _ = launch(ctx, a, b, c0, m, n, k, ty, batch=batch, strides=(sa, sb, sc), label="batched")
+    for got, z in itertools.product(results, range(batch)):
         hi, lo, ab = oracle.ref_gemm_wide(a[z * sa:], b[z * sb:], m, n, k)
         assert oracle.check_wide(got[z * sc:z * sc + m * n].reshape(m, n), hi, lo, ab, k) <= 1.0
         assert np.array_equal(got[z * sc + m * n:(z + 1) * sc].view(np.uint8), c0[z * sc + m * n:(z + 1) * sc].view(np.uint8))
@@ -208,12 +219,13 @@ def test_large_on_sampled_rows(ctx, oracle, ty, size):
     rng = np.random.default_rng(6)
     a = (rng.random(m * k) * 2 - 1).astype(dt)
     b = (rng.random(k * n) * 2 - 1).astype(dt)
-    got, _ = launch(ctx, a, b, np.zeros(m * n, dt), m, n, k, ty, label="large")
+    results, _ = launch(ctx, a, b, np.zeros(m * n, dt), m, n, k, ty, label="large")
     rows = np.unique(np.concatenate([[0, 1, 127, 128, m - 1], rng.integers(0, m, 43)])).astype(np.uint32)
     hi, lo, ab = oracle.ref_gemm_wide(a, b, m, n, k, rows=rows)
-    worst = oracle.check_wide(got.reshape(m, n)[rows], hi, lo, ab, k)
-    _say(f"large {ty}: worst error / bound = {worst:.3f}")
-    assert worst <= 1.0
+    for got in results:
+        worst = oracle.check_wide(got.reshape(m, n)[rows], hi, lo, ab, k)
+        _say(f"large {ty}: worst error / bound = {worst:.3f}")
+        assert worst <= 1.0
 
 
 def test_rejections(ctx):

@@ -301,40 +301,43 @@ def test_skinny_k_ranges_of_unequal_length(ctx, oracle, shape, ks):
     if ctx.info()["compute_units"] == 256:
         assert p["ksplit"] == ks
     a, b = mz.gen.normal_bf16(m * k, mz.gen.SEED_A, 1.0), mz.gen.normal_bf16(k * n, mz.gen.SEED_B, 0.02)
-    got = run_gemm(ctx, a, b, m, n, k)
+    got = run_gemm(ctx, a, b, m, n, k, kernel=p["kernel"])
     s = check_against_oracle(oracle, got, a, b, m, n, k, label=f"skinny {ks} ranges")
     _say(f"skinny {m}x{n}x{k} in {p['ksplit']} ranges {s}")
-    assert np.array_equal(got, run_gemm(ctx, a, b, m, n, k))                      # the tickets are back at zero, same bits
+    assert np.array_equal(got, run_gemm(ctx, a, b, m, n, k, kernel=p["kernel"]))  # the tickets are back at zero, same bits
+    form = mz.gemm_form(d, compute_units=ctx.info()["compute_units"])             # the launcher's own choice: the same ranges, the same bits
+    assert (form or p)["ksplit"] == p["ksplit"] and np.array_equal(got, run_gemm(ctx, a, b, m, n, k))
 
 
-def test_skinny_split_k_repeats_streams_and_batches(ctx, oracle):
+@pytest.mark.parametrize("kernel", [None, "maize_gemm_bf16_skinny_nn"])
+def test_skinny_split_k_repeats_streams_and_batches(ctx, oracle, kernel):
     """The M <= 16 kernel combines K ranges through a library-owned workspace whose ticket counters it
     must leave at zero: repeated launches, launches on another stream and batched launches all have to
     give the same bits."""
     m, n, k = 16, 1096, 4096                      # 5 slabs -> the dispatcher splits K
     a = mz.gen.normal_bf16(m * k, mz.gen.SEED_A, 1.0)
     b = mz.gen.normal_bf16(k * n, mz.gen.SEED_B, 0.02)
-    first = run_gemm(ctx, a, b, m, n, k)
+    first = run_gemm(ctx, a, b, m, n, k, kernel=kernel)
     check_against_oracle(oracle, first, a, b, m, n, k, label="skinny split-K")
     for _ in range(3):
-        assert np.array_equal(run_gemm(ctx, a, b, m, n, k), first)
+        assert np.array_equal(run_gemm(ctx, a, b, m, n, k, kernel=kernel), first)
     for _ in range(3):                            # a destroyed stream takes its workspace with it: a recycled handle starts clean
         s = ctx.stream()
-        assert np.array_equal(run_gemm(ctx, a, b, m, n, k, stream=s), first)
+        assert np.array_equal(run_gemm(ctx, a, b, m, n, k, stream=s, kernel=kernel), first)
         ctx.stream_destroy(s)
     # a different shape in between (its workspace layout differs), then the first one again
     a2 = mz.gen.normal_bf16(7 * 2048, 3, 1.0)
     b2 = mz.gen.normal_bf16(2048 * 264, 4, 0.02)
-    got2 = run_gemm(ctx, a2, b2, 7, 264, 2048)
+    got2 = run_gemm(ctx, a2, b2, 7, 264, 2048, kernel=kernel)
     check_against_oracle(oracle, got2, a2, b2, 7, 264, 2048, label="skinny 7x264x2048")
-    assert np.array_equal(run_gemm(ctx, a, b, m, n, k), first)
+    assert np.array_equal(run_gemm(ctx, a, b, m, n, k, kernel=kernel), first)
     # batched: every member equals its single launch
     batch = 3
     ab = mz.gen.normal_bf16(batch * m * k, 5, 1.0)
     bb = mz.gen.normal_bf16(batch * k * n, 6, 0.02)
-    dense = run_gemm(ctx, ab, bb, m, n, k, batch=batch)
+    dense = run_gemm(ctx, ab, bb, m, n, k, batch=batch, kernel=kernel)
     for i in range(batch):
-        single = run_gemm(ctx, ab[i * m * k:(i + 1) * m * k], bb[i * k * n:(i + 1) * k * n], m, n, k)
+        single = run_gemm(ctx, ab[i * m * k:(i + 1) * m * k], bb[i * k * n:(i + 1) * k * n], m, n, k, kernel=kernel)
         assert np.array_equal(single, dense[i * m * n:(i + 1) * m * n])
 
 

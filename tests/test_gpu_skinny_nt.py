@@ -57,10 +57,11 @@ def test_every_8bit_encoding_through_the_skinny_kernel(ctx, oracle):
         a = np.resize(finite, m * k).reshape(m, k).astype(np.uint8)
         eye = np.zeros((k, k), dtype=np.uint8)
         eye[np.arange(k), np.arange(k)] = oracle.fp8_bits_from_f64(np.array([1.0]), elem)[0]
-        got, took = launch(ctx, a.ravel(), eye.ravel(), np.zeros(m * k, np.uint16), m, k, k, NT, fmt, k, k, k)
+        results, took = launch(ctx, a.ravel(), eye.ravel(), np.zeros(m * k, np.uint16), m, k, k, NT, fmt, k, k, k, forms_too=True)
         assert took == f"maize_gemm_{fmt}_skinny_nt"
         want = oracle.bf16_bits_from_f64(oracle.fp8_bits_to_f64(a, elem))
-        assert np.array_equal(oracle.bf16_bits_to_f64(got), oracle.bf16_bits_to_f64(want.ravel()))
+        for got in results:
+            assert np.array_equal(oracle.bf16_bits_to_f64(got), oracle.bf16_bits_to_f64(want.ravel()))
 
 
 def test_repeats_batches_and_the_shared_workspace(ctx, oracle):
@@ -70,18 +71,21 @@ def test_repeats_batches_and_the_shared_workspace(ctx, oracle):
     m, n, k = 16, 1096, 4096
     a = f8_uniform(oracle, m * k, 51, elem)
     b = f8_uniform(oracle, n * k, 52, elem)
-    first, took = launch(ctx, a, b, np.zeros(m * n, np.uint16), m, n, k, NT, "e4m3", k, k, n)
-    assert took == "maize_gemm_e4m3_skinny_nt"
-    for _ in range(3):
-        again, _ = launch(ctx, a, b, np.full(m * n, 0x7FC0, np.uint16), m, n, k, NT, "e4m3", k, k, n)
-        assert np.array_equal(again, first)
+    name = "maize_gemm_e4m3_skinny_nt"
+    for kernel in (None, name):                                   # (the launcher runs a form in its place)
+        first, took = launch(ctx, a, b, np.zeros(m * n, np.uint16), m, n, k, NT, "e4m3", k, k, n, kernel=kernel)
+        assert took == name
+        for _ in range(3):
+            again, _ = launch(ctx, a, b, np.full(m * n, 0x7FC0, np.uint16), m, n, k, NT, "e4m3", k, k, n, kernel=kernel)
+            assert np.array_equal(again, first)
     batch, sa, sb, sc = 3, m * k + 64, n * k + 128, m * n + 16
     ab_ = f8_uniform(oracle, batch * sa, 53, elem)
     bb_ = f8_uniform(oracle, batch * sb, 54, elem)
-    dense, took = launch(ctx, ab_, bb_, np.zeros(batch * sc, np.uint16), m, n, k, NT, "e4m3", k, k, n, batch=batch, strides=(sa, sb, sc))
-    assert took == "maize_gemm_e4m3_skinny_nt"
+    dense, took = launch(ctx, ab_, bb_, np.zeros(batch * sc, np.uint16), m, n, k, NT, "e4m3", k, k, n, batch=batch, strides=(sa, sb, sc), kernel=name)
+    assert took == name == mz.gemm_plan(mz.gemm_ex_desc(*(mz.GlobalMatrix(p << 32, *s) for p, s in ((1, (m, k)), (2, (n, k)), (3, (m, n)))), layout=NT, batch=batch,
+                                                        stride_a=sa, stride_b=sb, stride_c=sc, in_type=mz.IN_E4M3))["kernel"]
     for i in range(batch):
-        single, _ = launch(ctx, ab_[i * sa:i * sa + m * k], bb_[i * sb:i * sb + n * k], np.zeros(m * n, np.uint16), m, n, k, NT, "e4m3", k, k, n)
+        single, _ = launch(ctx, ab_[i * sa:i * sa + m * k], bb_[i * sb:i * sb + n * k], np.zeros(m * n, np.uint16), m, n, k, NT, "e4m3", k, k, n, kernel=name)
         assert np.array_equal(single, dense[i * sc:i * sc + m * n]), i
         assert not dense[i * sc + m * n:(i + 1) * sc].any(), "wrote between batch members"
     assert run_ex(ctx, oracle, 16, 1096, 4096, label="NN skinny after NT") == "maize_gemm_bf16_skinny_nn"

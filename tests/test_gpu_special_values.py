@@ -67,6 +67,10 @@ FAMILIES = [
     ("maize_gemm_bf16_skinny_nt_m64", 50, 264, 4104, NT),
     ("maize_gemm_bf16_wave32", 33, 17, 65, NN),
     ("maize_gemm_bf16_wave32", 33, 17, 65, NT),
+    ("maize_gemm_bf16_t128_nn", 48, 8200, 1024, NN),
+    ("maize_gemm_bf16_mt256_nn_h128_gen", 1000, 1000, 1000, NN),
+    ("maize_gemm_bf16_mt256_nt_packed", 24, 257, 4100, NT),
+    # the launcher's choice: a registry kernel, and four of its own forms
     (None, 16, 14336, 4096, NN),
     (None, 48, 8200, 1024, NN),
     (None, 1000, 1000, 1000, NN),
@@ -202,15 +206,17 @@ def test_inf_nan_through_the_fp32_and_fp64_kernels(ctx, ty, layout):
     a[1, 3] = np.inf; a[m - 1, k - 1] = -np.inf; a[127, 31] = np.nan; a[2, :] = -0.0
     b[k - 1, n - 1] = np.inf; b[5, 128] = -np.inf; b[0, 7] = np.nan; b[:, 3] = -0.0
     bs = np.ascontiguousarray(b.T) if layout == NT else b
-    got, plan = launch(ctx, a.ravel(), bs.ravel(), np.zeros(m * n, dtype=dt), m, n, k, ty, layout, label="special values")
-    got = got.reshape(m, n)
+    results, _ = launch(ctx, a.ravel(), bs.ravel(), np.zeros(m * n, dtype=dt), m, n, k, ty, layout, label="special values")
+    assert len(results) == 2                                          # the form and the registry kernel
     with np.errstate(invalid="ignore", over="ignore"):
         ref = a.astype(np.longdouble) @ b.astype(np.longdouble)
         ab = np.abs(a).astype(np.longdouble) @ np.abs(b).astype(np.longdouble)
-    assert np.array_equal(np.isnan(got), np.isnan(ref)), "NaN sets differ"
-    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref)), "Inf sets differ"
     fin = np.isfinite(ref)
     u = 2.0 ** -24 if ty == "f32" else 2.0 ** -53
-    err = np.abs(got[fin].astype(np.longdouble) - ref[fin])
     assert np.isnan(ref).sum() > 0 and np.isinf(ref).sum() > 0 and fin.sum() > 0
-    assert np.all(err <= (k / 4.0 + 4.0) * u * ab[fin] + 1e-300), float((err / ((k / 4.0 + 4.0) * u * ab[fin] + 1e-300)).max())
+    for got in results:
+        got = got.reshape(m, n)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), "NaN sets differ"
+        assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref)), "Inf sets differ"
+        err = np.abs(got[fin].astype(np.longdouble) - ref[fin])
+        assert np.all(err <= (k / 4.0 + 4.0) * u * ab[fin] + 1e-300), float((err / ((k / 4.0 + 4.0) * u * ab[fin] + 1e-300)).max())

@@ -34,7 +34,8 @@ def _both(ctx, m, n, k, layout=mz.LAYOUT_NN, dist="normal"):
             try:
                 desc = mz.gemm_desc(mz.Matrix(da, m, k), mz.Matrix(db, k, n) if layout == mz.LAYOUT_NN else mz.Matrix(db, n, k),
                                     mz.Matrix(dc, m, n, offset_elems=PAD), layout=layout)
-                plan = mz.gemm_plan(desc, compute_units=ctx.info()["compute_units"])
+                cus = ctx.info()["compute_units"]
+                plan = mz.gemm_form(desc, compute_units=cus) or mz.gemm_plan(desc, compute_units=cus)      # what runs
                 _say(f"noalloc: {m}x{n}x{k} layout={layout} entry={'noalloc' if noalloc else 'alloc'} kernel={plan['kernel']} "
                      f"ksplit={plan['ksplit']} workspace={plan['workspace_bytes']}")
                 if noalloc:
@@ -65,12 +66,13 @@ def test_noalloc_matches_the_allocating_entry_point_twice_in_a_row(ctx, oracle):
         oracle.assert_parity(s, "noalloc")
 
 
-@pytest.mark.parametrize("shape", [(64, 4096, 4096, mz.LAYOUT_NN), (16, 4096, 4096, mz.LAYOUT_NT), (4000, 4120, 4032, mz.LAYOUT_NN),
-                                   (512, 512, 512, mz.LAYOUT_NN)],
-                         ids=["splitk_mt256", "skinny_nt", "edge_split", "no_scratch_needed"])
+@pytest.mark.parametrize("shape", [(96, 8192, 8192, mz.LAYOUT_NN, "_splitk"), (16, 28672, 1024, mz.LAYOUT_NT, "skinny_nt"), (4000, 4120, 4032, mz.LAYOUT_NN, "_edge"),
+                                   (64, 4096, 4096, mz.LAYOUT_NN, "maize_tile_"), (16, 4096, 4096, mz.LAYOUT_NT, "maize_tile_"), (512, 512, 512, mz.LAYOUT_NN, None)],
+                         ids=["splitk_mt256", "skinny_nt", "edge_split", "form_nn", "form_nt", "no_scratch_needed"])
 def test_noalloc_every_scratch_user(ctx, shape):
-    m, n, k, layout = shape
+    m, n, k, layout, kernel = shape
     ref, got, plan, _, _ = _both(ctx, m, n, k, layout=layout, dist="uniform")
+    assert (plan["workspace_bytes"] > 0) == (kernel is not None) and (kernel or "") in plan["kernel"], plan
     assert np.array_equal(ref, got), f"{plan['kernel']}: {int((ref != got).sum())} elements differ"
 
 
