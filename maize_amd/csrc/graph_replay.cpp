@@ -1,5 +1,5 @@
 // A caller that cannot allocate: a chain of products through maize_hip_gemm_bf16_noalloc, captured once into a HIP
-// graph on the caller's own stream and replayed with new inputs.  Every product in the chain passes partial tiles
+// graph on the caller's own stream and replayed with new inputs.  All products in the chain but one pass partial tiles
 // and ticket counters through the library's fixed per-GPU scratch array; every replay must reproduce, bit for bit,
 // what the same calls give when launched eagerly on the same inputs -- the kernels return their counters to zero
 // themselves, and nothing on the path allocates, synchronises or records a memset node.  (The reference has no
@@ -33,11 +33,12 @@ int main(int argc, char** argv) {
     MZ_OK(maize_hip_ctx_create(0, &ctx));
     // a few-row product in K ranges, the same against N x K weights, 64 rows in four row groups (the slab's workgroups
     // share the additions), 128-row tiles cut over K with the reduce pass behind them, a ragged product (24 columns past the last whole tile column) whose edge tiles
-    // are split, and a plain one that needs no scratch
-    std::vector<Product> ps = {{16, 14336, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {16, 4096, 4096, MAIZE_LAYOUT_NT, nullptr, nullptr, nullptr, {}, ""},
-                               {64, 14336, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {100, 2048, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""},
-                               {4000, 4120, 512, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {512, 512, 512, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}};
-    int with_scratch = 0;
+    // are split; then the launcher's own forms: two in K ranges, and one that needs no scratch
+    std::vector<Product> ps = {{16, 14336, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {16, 28672, 1024, MAIZE_LAYOUT_NT, nullptr, nullptr, nullptr, {}, ""},
+                               {64, 14336, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {96, 8192, 8192, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""},
+                               {4000, 4120, 512, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {16, 4096, 4096, MAIZE_LAYOUT_NT, nullptr, nullptr, nullptr, {}, ""},
+                               {100, 2048, 4096, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}, {512, 512, 512, MAIZE_LAYOUT_NN, nullptr, nullptr, nullptr, {}, ""}};
+    int with_scratch = 0, launches = 0;
     for (Product& p : ps) {
         MZ_OK(maize_hip_malloc(ctx, (size_t)p.m * p.k * 2, (void**)&p.a));
         MZ_OK(maize_hip_malloc(ctx, (size_t)p.k * p.n * 2, (void**)&p.b));
@@ -48,13 +49,18 @@ int main(int argc, char** argv) {
         p.desc.c = {p.c, p.m, p.n};
         p.desc.layout = p.layout;
         p.desc.batch = 1;
-        maize_gemm_plan_t plan;
-        MZ_OK(maize_hip_gemm_plan(&p.desc, nullptr, 256, &plan));
-        char name[96];
-        MZ_OK(maize_hip_gemm_select(ctx, &p.desc, name, sizeof name));
-        p.kernel = name;
-        with_scratch += plan.workspace_bytes > 0;
-        if (plan.workspace_bytes > MAIZE_NOALLOC_MAX_WORKSPACE_BYTES) { fprintf(stderr, "%s needs too much scratch\n", name); return 2; }
+        maize_gemm_ex_desc_t x;
+        std::memset(&x, 0, sizeof x);
+        x.gemm = p.desc;
+        x.alpha = 1.0f;
+        maize_gemm_plan_t plan, form;
+        MZ_OK(maize_hip_gemm_ex_plan(&x, nullptr, 256, &plan));
+        MZ_OK(maize_hip_gemm_ex_form(&x, 256, &form));
+        if (plan.workspace_bytes > MAIZE_NOALLOC_MAX_WORKSPACE_BYTES) { fprintf(stderr, "%s needs too much scratch\n", plan.kernel); return 2; }
+        const maize_gemm_plan_t& runs = form.kernel[0] ? form : plan;
+        p.kernel = runs.kernel;
+        with_scratch += runs.workspace_bytes > 0;
+        launches += 1 + (runs.reduce_grid > 0);
     }
     auto fill = [&](uint64_t seed) -> int {
         for (size_t i = 0; i < ps.size(); ++i) {
@@ -137,9 +143,9 @@ int main(int argc, char** argv) {
     HIP_OK(hipEventElapsedTime(&ms_eager, e0, e1));
     std::string names;
     for (const Product& p : ps) names += (names.empty() ? "\"" : ", \"") + p.kernel + "\"";
-    printf("{\"products\": %zu, \"with_scratch\": %d, \"graph_nodes\": %zu, \"rounds\": %d, \"mismatches\": %llu, \"us_per_chain_graph\": %.1f, "
+    printf("{\"products\": %zu, \"with_scratch\": %d, \"launches\": %d, \"graph_nodes\": %zu, \"rounds\": %d, \"mismatches\": %llu, \"us_per_chain_graph\": %.1f, "
            "\"us_per_chain_eager\": %.1f, \"kernels\": [%s]}\n",
-           ps.size(), with_scratch, nodes, rounds, (unsigned long long)mismatches, ms_graph / reps * 1e3, ms_eager / reps * 1e3, names.c_str());
+           ps.size(), with_scratch, launches, nodes, rounds, (unsigned long long)mismatches, ms_graph / reps * 1e3, ms_eager / reps * 1e3, names.c_str());
     HIP_OK(hipGraphExecDestroy(exec));
     HIP_OK(hipGraphDestroy(graph));
     HIP_OK(hipStreamDestroy(stream));
