@@ -1,5 +1,6 @@
 """The launcher's own forms without a device: what their code object contains, and the LDS layouts they add."""
 import os
+import random
 import re
 import shutil
 import subprocess
@@ -115,3 +116,67 @@ def test_no_register_that_a_fragment_read_is_still_filling_is_touched():
                 reads += 1
                 filling |= regs(args.split(",")[0])
     assert reads > 1000 and not early, early[:8]
+
+
+SIZE = {mz.IN_BF16: 2, mz.IN_F16: 2, mz.IN_E4M3: 1, mz.IN_E5M2: 1, mz.IN_E4M3_E5M2: 1, mz.IN_E5M2_E4M3: 1, mz.IN_F32: 4, mz.IN_F64: 8}
+TAG = {mz.IN_BF16: "bf16", mz.IN_F16: "f16", mz.IN_E4M3: "e4m3", mz.IN_E5M2: "e5m2", mz.IN_E4M3_E5M2: "e4m3e5m2", mz.IN_E5M2_E4M3: "e5m2e4m3", mz.IN_F32: "f32", mz.IN_F64: "f64"}
+
+
+def describe(m, n, k, nt=False, in_type=mz.IN_BF16, batch=1, **how):
+    a, b, c = (mz.GlobalMatrix(p << 44, *s) for p, s in ((1, (m, k)), (2, (n, k) if nt else (k, n)), (3, (m, n))))
+    return mz.gemm_ex_desc(a, b, c, layout=mz.LAYOUT_NT if nt else mz.LAYOUT_NN, batch=batch, in_type=in_type, stride_a=m * k, stride_b=k * n, stride_c=m * n, **how)
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_what_a_form_is_launched_with(seed):
+    """Drawn products: the grid covers C once per K range and fits a launch, no range is empty, workspace and ticket counters hold
+    what the kernel addresses, 8-bit operands are widened where the plan's kernel widens them and nowhere else, and the few-row
+    kernels' K ranges are kept."""
+    rng = random.Random(seed)
+    taken = split = pinned = 0
+    for i in range(3600):
+        m, n, k = (max(1, int(2 ** rng.uniform(0, hi)) // g * g) for hi, g in ((rng.choice([6, 13]), rng.choice([1, 8])), (15, rng.choice([1, 8, 16, 64])), (14, rng.choice([1, 8, 16, 64]))))
+        in_type, nt, batch, cus = rng.choice(list(SIZE)), rng.random() < 0.5, rng.choice([1, 1, 1, 3, 40]), rng.choice([256, 256, 304, 64, 1])
+        if i >= 3000:                                            # few rows against a row-major B
+            m, n, k, in_type, nt = rng.randint(1, 64), int(2 ** rng.uniform(8, 15)), 32 * rng.randint(8, 256), rng.choice([mz.IN_BF16, mz.IN_F16]), False
+        x = describe(m, n, k, nt, in_type, batch)
+        form, plan = mz.gemm_form(x, cus), mz.gemm_plan(x, compute_units=cus)
+        if form is None:
+            continue
+        es = SIZE[in_type]
+        got = re.fullmatch(r"maize_tile_([a-z0-9]+)_(nn|nt)_(\d+)x(\d+)(w?)", form["kernel"])
+        assert got and got[1] == TAG[in_type] and got[2] == ("nt" if nt else "nn"), form
+        bm, bn, ks = int(got[3]), int(got[4]), form["ksplit"]
+        tiles, steps = -(-m // bm) * -(-n // bn) * batch, -(-k * es // 128)
+        assert form["grid"] == (tiles * ks, 1, 1) and form["block"] == (256, 1, 1) and tiles * ks < 1 << 24
+        assert bool(got[5]) == (es == 1 and "_wave32" in plan["kernel"])
+        assert k * es >= 16 and (nt or n * es >= 16)
+        taken += 1
+        if ks == 1:
+            assert form["workspace_bytes"] == 0
+        else:
+            per = -(-steps // ks)
+            assert (ks - 1) * per < steps and tiles <= 16384
+            assert form["workspace_bytes"] == 65536 + tiles * ks * bm * bn * (8 if es == 8 else 4) < 1 << 32
+            split += 1
+        if "_skinny_nn" in plan["kernel"] and es == 2:
+            pinned += 1
+            assert ks == max(1, plan["ksplit"]) and (ks == 1 or -(-(-(-k // 32)) // ks) * 32 == -(-steps // ks) * 64)
+    assert taken > 1000 and split > 200 and pinned > 20, (taken, split, pinned)
+
+
+@pytest.mark.parametrize("in_type", list(SIZE), ids=list(TAG.values()))
+def test_where_no_form_can_run(in_type):
+    """Less than one 16-byte chunk of K, or of a row of a row-major B; extents and leading dimensions of 2^21 elements."""
+    ch = 16 // SIZE[in_type]
+    for nt in (False, True):
+        assert mz.gemm_form(describe(40, 50, ch, nt, in_type)) is not None
+        assert ch == 1 or mz.gemm_form(describe(40, 50, ch - 1, nt, in_type)) is None
+        assert (mz.gemm_form(describe(40, ch - 1, 50, nt, in_type)) is None) == (not nt)
+        assert mz.gemm_form(describe(40, ch, 50, nt, in_type)) is not None
+        for ld in ("lda", "ldb", "ldc"):
+            assert mz.gemm_form(describe(40, 50, 60, nt, in_type, **{ld: (1 << 21) - 1})) is not None
+            try:
+                assert mz.gemm_form(describe(40, 50, 60, nt, in_type, **{ld: 1 << 21})) is None
+            except mz.MaizeError:                                # (some are refused altogether: there is one fp64 kernel)
+                assert in_type == mz.IN_F64
