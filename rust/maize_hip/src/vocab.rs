@@ -143,7 +143,12 @@ impl DescribedGemm {
     pub fn launch(&self, ctx: &Ctx, stream: *mut core::ffi::c_void) -> Result<()> {
         let mut info: ffi::MaizeDeviceInfo = unsafe { core::mem::zeroed() };
         let cus = if unsafe { ffi::maize_hip_device_info(ctx.handle(), &mut info) } == ffi::MAIZE_OK { info.compute_units } else { 256 };
-        let forced = self.described_kernel(cus)?;
+        let mut forced = self.described_kernel(cus)?;
+        let mut form: ffi::MaizeGemmPlan = unsafe { core::mem::zeroed() };
+        if forced.is_none() && unsafe { ffi::maize_hip_gemm_ex_form(&self.desc, cus, &mut form) } == ffi::MAIZE_OK && form.kernel[0] != 0 {
+            // the dispatcher's choice is of the described family; unnamed, the form would run
+            forced = plan_of(&self.desc, None, cus).and_then(|k| std::ffi::CString::new(k).ok());
+        }
         let rc = unsafe { ffi::maize_hip_gemm_bf16_ex(ctx.handle(), &self.desc, forced.as_ref().map_or(core::ptr::null(), |k| k.as_ptr()), stream) };
         if rc == ffi::MAIZE_OK { Ok(()) } else { Err(Error { code: rc, message: "maize_hip_gemm_bf16_ex".into() }) }
     }
