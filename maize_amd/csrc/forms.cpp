@@ -41,7 +41,7 @@ const Names& names() {
 // what does not fit the memory-side cache comes from HBM; residuals 8-14 %):
 //   t0 + core + [K tail] tail + [K ranges] (r0 + r1 * ranges)
 // core: `one` per K tile where a compute unit has one workgroup, `many` per K tile and workgroup where it has several (what
-// bounds them is the rate at which a compute unit's LDS is filled: 75-100 GB/s) and `turn` for each workgroup after the first;
+// bounds them is the rate at which a compute unit's requests arrive in its LDS: 75-100 GB/s) and `turn` for each workgroup after the first;
 // rows of A (B) that are no 16-byte material make the requests longer by ua (ub), transposing reads by nn, 8-bit
 // operands by e8; at least bytes / bw.
 struct TileCost { uint32_t bm, bn; double t0, one, many, turn, r0, r1, ua, ub, nn, bw, tail, e8; };

@@ -3,7 +3,7 @@
 //
 // They are to the registry what the tail split is: the same product, composed differently.  maize_hip_gemm_plan and
 // maize_hip_gemm_select keep reporting the registry kernel, whose requirements and arithmetic (8-bit operands: multiplied as
-// they are, or widened) the form shares.
+// they are, or widened) the form shares; maize_hip_gemm_ex_form reports the form.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>

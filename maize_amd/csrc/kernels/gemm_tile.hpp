@@ -18,8 +18,10 @@
 //     a pass of their own;
 //   * C goes through LDS and out in runs of eight columns, whatever its alignment (128-bit stores may start on any element).
 //
-// What bounds them: the rate at which a compute unit's LDS is filled, 75-100 GB/s (16, 20 or 24 KiB per K tile: 0.17-0.28 us
-// with one workgroup per compute unit), and some 3 us of launch, first loads and epilogue.  Tiles of 64 x 64 move twice the bytes
+// What bounds them: the rate at which a compute unit's requests arrive in its LDS, 75-100 GB/s (16, 20 or 24 KiB per K tile: 0.17-0.28
+// us with one workgroup per compute unit; 41 of the 64 bytes per cycle of the vector L1), and some 3 us of launch, first loads and
+// epilogue.  Counters (1024^3, 544 x 2472 x 1112, E4M3 16 x 14336 x 4096): matrix pipe busy 0.13-0.19 and LDS reads 0.15-0.18 of the
+// time, no bank conflicts, waves waiting 0.44-0.57.  Tiles of 64 x 64 move twice the bytes
 // of 128 x 128 per multiply-add but give four times the workgroups, two per compute unit at a time: 1024^3 11.2 -> 7.0 us, 256^3
 // 6.2 -> 4.5, 200 x 1072 x 368 9.9 -> 5.4; 64 x 128 where there are enough of them: 544 x 2472 x 1112 21.0 -> 11.3, 1632 x 1072 x
 // 1392 22.9 -> 12.8; 32 x 128 for few rows.  Ragged K against copies of the operands in the workspace: 1024 x 3072 x 1999 61.4 -> 25.9,
@@ -27,12 +29,13 @@
 // 128 x 168 x 296 63 -> 5.5.  (Tried and slower: twice the ring depth on one workgroup per compute unit, three stages on three.)
 //
 // 128 x 128 of 16- and 8-bit operands: what bounds the smaller tiles on a product of a round or two is the LDS fill, which this
-// halves per multiply-add.  One workgroup of four ring stages (128 KiB) per compute unit: two of two stages have too few
+// halves per multiply-add.  What bounds it in turn is one wave per SIMD (1024 x 3072 x 1999: waits 0.30, waits to issue 0.35, matrix pipe
+// 0.30).  One workgroup of four ring stages (128 KiB) per compute unit: two of two stages have too few
 // registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
 // 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
 //
 // fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
-// What bounds them is the matrix pipe: a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
+// What bounds them is the matrix pipe (busy 0.97 and 0.95 of the time at 4096^3): a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
 // A lane's 16-byte chunk feeds four (two) instructions in turn, the same k on both sides, so a K-contiguous operand needs an
 // eighth of the reads of one element per instruction, and the next K tile's reads run behind this one's instructions.  Against
 // 128 x 128 tiles copied through registers, whose reads stand in front of the instructions they feed: 2048^3 fp32 N x K 162.6 ->
