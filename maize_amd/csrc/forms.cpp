@@ -150,7 +150,7 @@ double registry_cost(const FamilyOf& f, const Problem& p, const LaunchDims& ld) 
         const double core = rounds * cdiv(p.steps, ks) * (nn ? 0.44 : 0.85);
         return (nn ? 3.5 : 1.0) + longer(core, p.bytes / (nn ? 6.35e6 : 5.33e6)) + (ks > 1u ? (nn ? 3.8 : 0.0) + (nn ? 0.19 : 0.65) * ks * groups : 0.0);
     }
-    // fp32 and fp64, and the any-shape kernel: the form always (choose_form)
+    // fp32 and fp64 (but for what choose_form keeps), and the any-shape kernel: the form always
     if (f.family == kAnyShape || f.family == kWide) return 1e9;
     if (f.family == kUnknown) return 0.0;                            // (a kernel that this table does not know keeps its products)
     const RegistryCost& c = kRegistryCost[f.family][p.esz == 1u];
@@ -201,8 +201,6 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     LaunchDims ld;
     std::memset(&ld, 0, sizeof ld);
     if (!kernel_at(registry).plan(d, compute_units, &ld)) return false;       // (what the registry's kernel refuses stays refused)
-    // fp32 and fp64: the form always.  The registry's 128 x 128 tiles through registers take 4.3 (fp64 5.7) times as long on the
-    // average of 2000 drawn products; they are more than 3 % ahead on 41, at most 24 %, most of them a short K with many tiles.
     const double rival = registry_cost(of, p, ld);
 
     // The any-shape kernel multiplies 8-bit operands widened to bf16: its form does too.  Everywhere else the other tiles.
@@ -234,6 +232,15 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
     }
     const TileCost& c = fam == kWide ? kFullCost[d.in_type - MAIZE_IN_F32][tile] : kTileCost[tile];
     const uint64_t tiles = (uint64_t)cdiv(p.s.m, c.bm) * cdiv(p.s.n, c.bn) * p.batch, items = tiles * ranges;
+    // fp32 and fp64: the registry's 128 x 128 tiles through registers take 4.3 (fp64 5.7) times as long on the average of 2000 drawn
+    // products.  They keep those that have so short a K and so many tiles that the form's are the same, or nearly, and its ring is
+    // mostly prologue, where all rows are 16-byte material (4096 x 15584 x 32 fp64 172.9 -> 143.8 us, 7203 x 17704 x 16 fp32 143.7 ->
+    // 120.6).  Of 3945 fp32 products (six tenths with K up to 512) the form is more than 3 % behind on 374 without this rule and
+    // on 57 with it; on 34 of the 449 that the rule keeps the registry's kernel is, by 10 % at most.  Of 2055 fp64 ones: 34, 20, 4 of 36.
+    if (fam == kWide && ld.split_first == 7u) {
+        const uint64_t tiles128 = (uint64_t)cdiv(p.s.m, 128) * cdiv(p.s.n, 128) * p.batch;
+        if (d.in_type == MAIZE_IN_F32 ? tile == T128x128 && p.steps <= 4u : p.steps <= 3u && tiles128 >= 8u * compute_units) return false;
+    }
     // The form has to win by the model; by 8 % against 128-row tiles and K ranges above 64 rows, by 10 % against the few-row kernels
     // (the shares that left the sum of all times least).  Of 4000 drawn products 3352 then run a form, in 0.47 of the registry
     // kernel's time on average; 42 of them are more than 3 % slower on it, 20 more than 10 %, at most 29 % (with one share of 0.9, and

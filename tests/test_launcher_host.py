@@ -223,6 +223,25 @@ def test_products_that_a_form_slows_down_stay_on_the_registry_kernel(dev, x):
     assert mz.gemm_form(x) is None and launches(dev.product(x))[-1].kernel.startswith("maize_")
 
 
+SHORT_K = [product(7203, 17704, 16, in_type=mz.IN_F32), product(1280, 3216, 8, in_type=mz.IN_F32, batch=8), product(8544, 7372, 32, nt=True, in_type=mz.IN_F32),
+           product(968, 4064, 112, in_type=mz.IN_F32, batch=32), product(4096, 15584, 32, nt=True, in_type=mz.IN_F64), product(240, 14280, 48, in_type=mz.IN_F64, batch=32)]
+
+
+@pytest.mark.parametrize("x", SHORT_K)
+def test_fp32_and_fp64_products_of_a_short_k_stay_on_the_registry_kernel(dev, x):
+    """(8 to 23 % slower on the form: its tiles are the same, or nearly, and the ring is mostly prologue.)"""
+    assert mz.gemm_form(x) is None
+    ran = launches(dev.product(x))
+    assert len(ran) == 1 and "_mt128_" in ran[0].kernel and ran[0].kernel == mz.gemm_plan(x)["kernel"]
+
+
+@pytest.mark.parametrize("x", [product(7203, 17704, 15, in_type=mz.IN_F32), product(7203, 17702, 16, in_type=mz.IN_F32), product(1280, 3216, 8, in_type=mz.IN_F32, ldc=3217),
+                               product(1280, 3216, 132, in_type=mz.IN_F32, batch=8), product(64, 3216, 16, in_type=mz.IN_F32), product(1024, 4096, 32, in_type=mz.IN_F64)])
+def test_the_other_fp32_and_fp64_products_run_a_form(dev, x):
+    """Rows that are no 16-byte material, a K tile more, fewer tiles."""
+    assert "maize_tile_f" in mz.gemm_form(x)["kernel"]
+
+
 def test_every_registry_kernel_has_a_cost(tmp_path):
     """A kernel whose name the cost model does not know would keep all its products; none does, and the table has a row for it."""
     src = tmp_path / "families.cpp"
