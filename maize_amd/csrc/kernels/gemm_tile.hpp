@@ -30,9 +30,18 @@
 //
 // 128 x 128 of 16- and 8-bit operands: what bounds the smaller tiles on a product of a round or two is the LDS fill, which this
 // halves per multiply-add.  What bounds it in turn is one wave per SIMD (1024 x 3072 x 1999: waits 0.30, waits to issue 0.35, matrix pipe
-// 0.30).  One workgroup of four ring stages (128 KiB) per compute unit: two of two stages have too few
+// 0.30).  One workgroup of five ring stages (the 160 KiB) per compute unit: two of two stages have too few
 // registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
 // 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
+//
+// Five ring stages (64 x 64, and 128 x 128 of 16- and 8-bit operands): requests in pairs of K tiles.  Rows that do not start on
+// 128-byte lines -- any K that is no multiple of a K tile's -- have every K tile's 128 bytes of a row on two lines, and what
+// bounds these tiles is the rate at which lines reach a compute unit (about 100 GB/s; a fifth stage alone changed
+// nothing, 1700 x 2000 x 4999 57.0 us with four and 57.4 with five).  The lines that two K tiles of a row share are drawn
+// once if both are asked for together: three lines instead of four.  Two stages are free for it in every other step if the ring
+// has five: even steps ask for A of two K tiles, odd ones for B.  N x K, bf16: 1700 x 2000 x 4999 57.0 -> 51.8 us (596 ->
+// 656 TFLOP/s), 1024 x 3072 x 2047 26.7 -> 25.2; K x N, where only A's lines are shared, 49.7 -> 46.8 and 22.5 -> 22.1; 64 x 64
+// tiles, 150 x 201 x 333 5.95 -> 5.43, 2096 x 992 x 1184 N x K 16.6 -> 16.4.
 //
 // fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
 // What bounds them is the matrix pipe (busy 0.97 and 0.95 of the time at 4096^3): a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
@@ -239,6 +248,8 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     constexpr int PA = BM / 32, PB = BN / 32, P = PA + PB;            // 1 KiB requests per wave and K tile
     constexpr uint32_t ASTAGE = BM * 128u, BSTAGE = BN * 128u;
     typedef KN<ES, BN> KNB;
+    // The requests of two K tiles of one operand go out together, a row of the one next to the same row of the other (above).
+    constexpr bool PAIR = !FP && NS == 5;
     static_assert(NS * (BM + BN) * 128u >= BM * BN * AS, "the epilogue's fp32 tile takes the ring's place");
     __shared__ __attribute__((aligned(1024))) char lds_a[NS * (ASTAGE + BSTAGE)];
     char* const lds_b = lds_a + NS * ASTAGE;
@@ -326,6 +337,11 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
 #pragma unroll
         for (int q = 0; q < P; ++q) piece(r, q);
     };
+    auto request_pair = [&](uint32_t s, uint32_t st) {                // entries s and s + 1 into stages st and st + 1
+        const TileReq r = tile_req(s, st), r2 = tile_req(s + 1u, st + 1u);
+#pragma unroll
+        for (int q = 0; q < P; ++q) { piece(r, q); piece(r2, q); }
+    };
 
     accx4 acc[MI][NJ];
 #pragma unroll
@@ -373,8 +389,15 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
             else    put(at, tb[i], n0 + KNB::chunk(pc, lane) * CH, N - CH, k_main + KNB::row(pc, lane) < K);
         }
     };
-    const uint32_t primed = nd < (uint32_t)NS ? nd : (uint32_t)NS;
-    for (uint32_t s = 0; s < primed; ++s) request(s, s);
+    constexpr uint32_t PRIME = PAIR ? 4u : (uint32_t)NS;
+    const uint32_t primed = nd < PRIME ? nd : PRIME;
+    if constexpr (PAIR) {
+        uint32_t s = 0;
+        for (; s + 1u < primed; s += 2u) request_pair(s, s);
+        if (s < primed) request(s, s);
+    } else {
+        for (uint32_t s = 0; s < primed; ++s) request(s, s);
+    }
     if (tail_here && nd < (uint32_t)NS) place_tail(nd);
     // Waits until all but the youngest `n` entries' requests of this wave have landed, then for the other waves.
     auto meet = [&](uint32_t n) {
@@ -384,7 +407,7 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
         });
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     };
-    meet(primed ? primed - 1u : 0u);
+    meet(PAIR ? (primed > 2u ? primed - 2u : 0u) : primed ? primed - 1u : 0u);
 
     // Fragment reads (maps.hpp): one base per K half (K-contiguous tiles; fragment f sits 2048 f bytes further on) or per
     // column group (K x N tile).
@@ -468,16 +491,33 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
         else if constexpr (!WIDE) mfma8<(ET - 2) & 1, ((ET - 2) >> 1)>(acc[i][j], b_half(set, j, 0), b_half(set, j, 1), fa[S][i][0], fa[S][i][1]);
     };
     uint32_t st = 0u;                                                 // ring stage of the entry in hand
+    uint32_t left = 0u;                                               // an entry without a partner is on its way
     auto step = [&](auto set, auto requests, uint32_t s) {            // 2: requests entry s + NS; 1: if there is one (or places the tail); 0: there is none
         constexpr int S = decltype(set)::value;
         constexpr int REQ = decltype(requests)::value;
         constexpr std::integral_constant<int, 1 - S> other{};
-        if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((NS - 2) * P) : "memory");
+        if constexpr (PAIR) {
+            // entry s + 1 landed with entry s (S = 0), or all but the youngest requests (of A: two entries' ahead of it) have
+            if constexpr (S == 0 && REQ != 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(2 * PA) : "memory");
+            else meet(REQ == 1 ? left : 0u);
+        }
+        else if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"((NS - 2) * P) : "memory");
         else meet(nd < s + 2u ? 0u : nd - s - 2u < (uint32_t)NS - 2u ? nd - s - 2u : (uint32_t)NS - 2u);
         const uint32_t nst = st + 1u == (uint32_t)NS ? 0u : st + 1u, ao = nst * ASTAGE, bo = nst * BSTAGE;
-        TileReq r;
-        if constexpr (REQ == 2) r = tile_req(s + (uint32_t)NS, st);
-        if constexpr (REQ == 1) {
+        TileReq r, r2;
+        constexpr int RP = !PAIR ? P : S == 0 ? 2 * PA : 2 * PB;      // requests of this step
+        const uint32_t pst = st ? st - 1u : (uint32_t)NS - 1u;        // (the stage of entry s - 1 is free, too)
+        if constexpr (REQ == 2 && PAIR) {
+            if constexpr (S == 0) { r = tile_req(s + 4u, pst); r2 = tile_req(s + 5u, st); }
+            else                  { r = tile_req(s + 3u, pst ? pst - 1u : (uint32_t)NS - 1u); r2 = tile_req(s + 4u, pst); }
+        }
+        else if constexpr (REQ == 2) r = tile_req(s + (uint32_t)NS, st);
+        if constexpr (REQ == 1 && PAIR && S == 0) {
+            if (s + 4u < nd) { request(s + 4u, pst); left = 1u; }
+            if (tail_here && nd >= (uint32_t)NS) place_tail(s + 4u < nd ? st : pst);
+        }
+        else if constexpr (REQ == 1 && !PAIR) {
             if (s + (uint32_t)NS < nd) request(s + (uint32_t)NS, st);
             else if (tail_here && s + (uint32_t)NS == nd) place_tail(st);
         }
@@ -490,7 +530,10 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
             });
             if constexpr (REQ == 2) {
 #pragma unroll
-                for (int q = n * P / NM; q < (n + 1) * P / NM; ++q) piece(r, q);
+                for (int q = n * RP / NM; q < (n + 1) * RP / NM; ++q) {
+                    if constexpr (PAIR) piece(q & 1 ? r2 : r, S * PA + q / 2);
+                    else piece(r, q);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -521,7 +564,7 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     each<NR>([&](auto q_) { read_one(S0, q_, 0u, 0u); });
     landed(S0);
     uint32_t s = 0;
-    for (; s + (uint32_t)NS + 1u < nd; s += 2u) {
+    for (; s + (PAIR ? 5u : (uint32_t)NS + 1u) < nd; s += 2u) {
         step(S0, TWO, s);
         step(S1, TWO, s + 1u);
     }
@@ -633,8 +676,8 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 4, 1) \
-    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 4, 1)
+    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 5, 1) \
+    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 5, 1)
 MAIZE_TILE_16(bf16, 0)
 MAIZE_TILE_16(f16, 1)
 #define MAIZE_TILE_8(tag, et) \
@@ -646,8 +689,8 @@ MAIZE_TILE_16(f16, 1)
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 4, 1) \
-    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 4, 1)
+    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 5, 1) \
+    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 5, 1)
 MAIZE_TILE_8(e4m3, 2)
 MAIZE_TILE_8(e5m2, 5)
 MAIZE_TILE_8(e4m3e5m2, 4)

@@ -201,3 +201,15 @@ def test_a_captured_form_in_k_ranges_equals_the_eager_one(ctx, warm):
     ctx.stream_destroy(other)
     for x in (da, db, dla, dlb, dc, dlc):
         x.free()
+
+
+@pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
+@pytest.mark.parametrize("op,tile", [("bf16", "64x64"), ("bf16", "128x128"), ("e4m3", "64x64"), ("e4m3", "64x64w"), ("e4m3", "128x128")])
+def test_k_tiles_requested_in_pairs(ctx, oracle, forms, op, tile, layout):
+    """One K tile to two rounds of the five ring stages, an odd one out and a ragged one behind: each count of entries that the
+    pairs, the one without a partner and the stage of the tail can meet."""
+    bm, bn = TILES[tile]
+    kt = 64 if op == "bf16" else 128
+    for entries in range(1, 13):
+        for more in (0, 9):
+            check_form(ctx, oracle, forms, op, tile, layout, bm - 3, bn + 5, entries * kt + more, off=entries % 2, pad=more % 2)
