@@ -34,14 +34,16 @@
 // registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
 // 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
 //
-// Five ring stages (64 x 64, and 128 x 128 of 16- and 8-bit operands): requests in pairs of K tiles.  Rows that do not start on
+// 128 x 128 of 16- and 8-bit operands has five ring stages for requests in pairs of K tiles.  Rows that do not start on
 // 128-byte lines -- any K that is no multiple of a K tile's -- have every K tile's 128 bytes of a row on two lines, and what
 // bounds these tiles is the rate at which lines reach a compute unit (about 100 GB/s; a fifth stage alone changed
 // nothing, 1700 x 2000 x 4999 57.0 us with four and 57.4 with five).  The lines that two K tiles of a row share are drawn
 // once if both are asked for together: three lines instead of four.  Two stages are free for it in every other step if the ring
-// has five: even steps ask for A of two K tiles, odd ones for B.  N x K, bf16: 1700 x 2000 x 4999 57.0 -> 51.8 us (596 ->
-// 656 TFLOP/s), 1024 x 3072 x 2047 26.7 -> 25.2; K x N, where only A's lines are shared, 49.7 -> 46.8 and 22.5 -> 22.1; 64 x 64
-// tiles, 150 x 201 x 333 5.95 -> 5.43, 2096 x 992 x 1184 N x K 16.6 -> 16.4.
+// has five: even steps ask for A of two K tiles, odd ones for B.  N x K, bf16: 1700 x 2000 x 4999 57.1 -> 52.0 us (595 ->
+// 654 TFLOP/s), 1024 x 3072 x 1999 30.1 -> 28.4, E4M3 928 x 2568 x 5992 35.4 -> 29.1; K x N, where only A's lines are shared,
+// 49.7 -> 46.8 and 22.5 -> 22.1.  Not the 64 x 64 tiles, which have five stages too but less to multiply behind their loads: four K
+// tiles in flight instead of five cost half 16 x 14336 x 4096 N x K 24.7 -> 30.8 us, 1024^3 6.8 -> 7.4 and E4M3 19 x 10987 x
+// 1494 6.7 -> 6.9 (and gave 150 x 201 x 333 5.95 -> 5.43, for its shorter code).
 //
 // fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
 // What bounds them is the matrix pipe (busy 0.97 and 0.95 of the time at 4096^3): a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
@@ -249,7 +251,7 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     constexpr uint32_t ASTAGE = BM * 128u, BSTAGE = BN * 128u;
     typedef KN<ES, BN> KNB;
     // The requests of two K tiles of one operand go out together, a row of the one next to the same row of the other (above).
-    constexpr bool PAIR = !FP && NS == 5;
+    constexpr bool PAIR = !FP && NS == 5 && BM == 128;
     static_assert(NS * (BM + BN) * 128u >= BM * BN * AS, "the epilogue's fp32 tile takes the ring's place");
     __shared__ __attribute__((aligned(1024))) char lds_a[NS * (ASTAGE + BSTAGE)];
     char* const lds_b = lds_a + NS * ASTAGE;
