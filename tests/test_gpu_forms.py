@@ -204,10 +204,11 @@ def test_a_captured_form_in_k_ranges_equals_the_eager_one(ctx, warm):
 
 
 @pytest.mark.parametrize("layout", [NN, NT], ids=["nn", "nt"])
-@pytest.mark.parametrize("op,tile", [("bf16", "64x64"), ("bf16", "128x128"), ("e4m3", "64x64"), ("e4m3", "64x64w"), ("e4m3", "128x128")])
-def test_k_tiles_requested_in_pairs(ctx, oracle, forms, op, tile, layout):
-    """One K tile to two rounds of the five ring stages, an odd one out and a ragged one behind: each count of entries that the
-    pairs, the one without a partner and the stage of the tail can meet."""
+@pytest.mark.parametrize("op,tile", [("bf16", "32x128"), ("bf16", "64x64"), ("bf16", "64x128"), ("bf16", "128x128"), ("e4m3", "32x128"), ("e4m3", "64x64"),
+                                     ("e4m3", "64x64w"), ("e4m3", "64x128"), ("e4m3", "128x128")])
+def test_every_count_of_k_tiles(ctx, oracle, forms, op, tile, layout):
+    """One K tile to two rounds of the three to five ring stages and a ragged one behind: each count of entries that the requests
+    (one by one or in pairs), the one without a partner and the stage of the tail can meet."""
     bm, bn = TILES[tile]
     kt = 64 if op == "bf16" else 128
     for entries in range(1, 13):
