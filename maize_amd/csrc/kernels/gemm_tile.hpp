@@ -34,16 +34,22 @@
 // registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
 // 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
 //
-// 128 x 128 of 16- and 8-bit operands has five ring stages for requests in pairs of K tiles.  Rows that do not start on
-// 128-byte lines -- any K that is no multiple of a K tile's -- have every K tile's 128 bytes of a row on two lines, and what
-// bounds these tiles is the rate at which lines reach a compute unit (about 100 GB/s; a fifth stage alone changed
-// nothing, 1700 x 2000 x 4999 57.0 us with four and 57.4 with five).  The lines that two K tiles of a row share are drawn
-// once if both are asked for together: three lines instead of four.  Two stages are free for it in every other step if the ring
-// has five: even steps ask for A of two K tiles, odd ones for B.  N x K, bf16: 1700 x 2000 x 4999 57.1 -> 52.0 us (595 ->
-// 654 TFLOP/s), 1024 x 3072 x 1999 30.1 -> 28.4, E4M3 928 x 2568 x 5992 35.4 -> 29.1; K x N, where only A's lines are shared,
-// 49.7 -> 46.8 and 22.5 -> 22.1.  Not the 64 x 64 tiles, which have five stages too but less to multiply behind their loads: four K
+// They ask for the K tiles of an operand in pairs, from five ring stages, where rows do not start on 128-byte lines: a K tile's
+// 128 bytes of a row are then on two lines, and the line that two K tiles share is read once if both are asked for together.
+// Reads from the L2: 8.57 -> 6.48 million of 1700 x 2000 x 4999 N x K, E4M3 928 x 2568 x 5992 3.69 -> 2.86, 1192 x 2580 x
+// 1856 (rows on lines) 1.474 both.  Single requests from four stages -> pairs: 1700 x 2000 x 4999 57.1 -> 52.0 us (595 ->
+// 654 TFLOP/s), E4M3 928 x 2568 x 5992 35.4 -> 29.1, 1024 x 3072 x 1999 K x N into fp32 25.4 -> 24.6, 96 drawn products 5 % off on
+// average and none longer.  Rows that do not start on dwords gain nothing (E4M3 1024 x 3072 x 1999 N x K 21.3 both): a request there is
+// about four accesses of the vector cache, which then bound the loop.
+// Rows on lines share nothing, and B is asked for one step later: 32 drawn products 2 % longer on average, 7 % at most (1192 x
+// 2580 x 1856 N x K 18.1 -> 19.1, E5M2 5176 x 2006 x 4096 51.2 -> 53.8, 1536 x 2203 x 4096 K x N 36.9 -> 38.5).  They have single requests and
+// four stages (with five, a K tile more stands in front of the first multiplication: 1 to 5 % longer as well); so have N x K products with one
+// operand on lines and one on half lines, which gain and lose 4 %.  One operand on lines and one anywhere: 1 to 5 % off on average, 2 %
+// longer at most; both on half lines, or A against a row-major B: 3 % off, 3 % longer at most.  The kernel looks at its operands
+// (maps::in_pairs).
+// Not the 64 x 64 tiles, which have five stages too but less to multiply behind their loads: four K
 // tiles in flight instead of five cost half 16 x 14336 x 4096 N x K 24.7 -> 30.8 us, 1024^3 6.8 -> 7.4 and E4M3 19 x 10987 x
-// 1494 6.7 -> 6.9 (and gave 150 x 201 x 333 5.95 -> 5.43, for its shorter code).
+// 1494 6.7 -> 6.9 (and gave 150 x 201 x 333 5.95 -> 5.43).
 //
 // fp32 and fp64 operands (v_mfma_f32_16x16x4_f32, v_mfma_f64_16x16x4_f64; no tf32 instruction exists): the same ring and tiles.
 // What bounds them is the matrix pipe (busy 0.97 and 0.95 of the time at 4096^3): a K tile of 128 bytes of a 64 x 64 tile is 1024 of its cycles against 16 KiB of LDS fill.
@@ -236,9 +242,10 @@ __device__ __forceinline__ bf16x8 widen8(uint32_t lo, uint32_t hi) {
 // ET: 0 bf16, 1 IEEE half, 2 + (A is E5M2) + 2 (B is E5M2): 8-bit operands, 6 fp32, 7 fp64.
 // WIDE: 8-bit operands widened to bf16 as their fragments are read (exact) and multiplied by the bf16 instruction: the
 // arithmetic of the any-shape kernel, which small 8-bit products get.
-// 4 waves as WM x WN, each MI x NJ accumulators of 16 x 16; NS ring stages.
-template <int ET, bool WIDE, bool NT, int BM, int BN, int NS>
-__device__ __forceinline__ void body(const GemmArgs& p) {
+// 4 waves as WM x WN, each MI x NJ accumulators of 16 x 16; NS ring stages in lds_a.
+// PAIR: the requests of two K tiles of one operand go out together, a row of the one next to the same row of the other (above).
+template <int ET, bool WIDE, bool NT, int BM, int BN, int NS, bool PAIR>
+__device__ __forceinline__ void body(const GemmArgs& p, char* lds_a) {
     constexpr bool IS8 = ET >= 2 && ET < 6, F16 = ET == 1, FP = ET >= 6;
     static_assert(!WIDE || IS8, "only 8-bit operands are widened");
     constexpr uint32_t ES = IS8 ? 1u : ET == 6 ? 4u : ET == 7 ? 8u : 2u, CH = 16u / ES, BKE = 128u / ES;
@@ -250,10 +257,8 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     constexpr int PA = BM / 32, PB = BN / 32, P = PA + PB;            // 1 KiB requests per wave and K tile
     constexpr uint32_t ASTAGE = BM * 128u, BSTAGE = BN * 128u;
     typedef KN<ES, BN> KNB;
-    // The requests of two K tiles of one operand go out together, a row of the one next to the same row of the other (above).
-    constexpr bool PAIR = !FP && NS == 5 && BM == 128;
+    static_assert(!PAIR || (NS == 5 && !FP), "two stages are free in every other step of a ring of five");
     static_assert(NS * (BM + BN) * 128u >= BM * BN * AS, "the epilogue's fp32 tile takes the ring's place");
-    __shared__ __attribute__((aligned(1024))) char lds_a[NS * (ASTAGE + BSTAGE)];
     char* const lds_b = lds_a + NS * ASTAGE;
     typedef __attribute__((address_space(3))) void* lvp;
 
@@ -667,10 +672,27 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     }
 }
 
+// 128 x 128 of 16- and 8-bit operands: in pairs where rows share lines between K tiles.
+template <int ET, bool NT>
+__device__ __forceinline__ void body_by_lines(const GemmArgs& p, char* lds) {
+    constexpr uint32_t ES = ET >= 2 ? 1u : 2u;
+    const auto off = [&](const void* x, uint32_t ld, uint64_t stride) { return maps::off_lines((uint64_t)(uintptr_t)x, ld * ES, p.batch > 1u ? stride * ES : 0u); };
+    if (maps::in_pairs(NT, off(p.a, lda_of(p), p.stride_a), off(p.b, ldb_of(p), p.stride_b))) body<ET, false, NT, 128, 128, 5, true>(p, lds);
+    else body<ET, false, NT, 128, 128, 4, false>(p, lds);
+}
+
 }  // namespace tile
 
 #define MAIZE_TILE(name, et, wide, nt, bm, bn, ns, perc) \
-    extern "C" __global__ __launch_bounds__(256, perc) void name(GemmArgs p) { tile::body<et, wide, nt, bm, bn, ns>(p); }
+    extern "C" __global__ __launch_bounds__(256, perc) void name(GemmArgs p) { \
+        __shared__ __attribute__((aligned(1024))) char lds[(ns) * ((bm) + (bn)) * 128]; \
+        tile::body<et, wide, nt, bm, bn, ns, false>(p, lds); \
+    }
+#define MAIZE_TILE_BY_LINES(name, et, nt) \
+    extern "C" __global__ __launch_bounds__(256, 1) void name(GemmArgs p) { \
+        __shared__ __attribute__((aligned(1024))) char lds[5 * (128 + 128) * 128]; \
+        tile::body_by_lines<et, nt>(p, lds); \
+    }
 #define MAIZE_TILE_16(tag, et) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x64, et, false, false, 64, 64, 5, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_64x64, et, false, true, 64, 64, 5, 2) \
@@ -678,8 +700,8 @@ __device__ __forceinline__ void body(const GemmArgs& p) {
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 5, 1) \
-    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 5, 1)
+    MAIZE_TILE_BY_LINES(maize_tile_##tag##_nn_128x128, et, false) \
+    MAIZE_TILE_BY_LINES(maize_tile_##tag##_nt_128x128, et, true)
 MAIZE_TILE_16(bf16, 0)
 MAIZE_TILE_16(f16, 1)
 #define MAIZE_TILE_8(tag, et) \
@@ -691,8 +713,8 @@ MAIZE_TILE_16(f16, 1)
     MAIZE_TILE(maize_tile_##tag##_nt_32x128, et, false, true, 32, 128, 4, 2) \
     MAIZE_TILE(maize_tile_##tag##_nn_64x128, et, false, false, 64, 128, 3, 2) \
     MAIZE_TILE(maize_tile_##tag##_nt_64x128, et, false, true, 64, 128, 3, 2) \
-    MAIZE_TILE(maize_tile_##tag##_nn_128x128, et, false, false, 128, 128, 5, 1) \
-    MAIZE_TILE(maize_tile_##tag##_nt_128x128, et, false, true, 128, 128, 5, 1)
+    MAIZE_TILE_BY_LINES(maize_tile_##tag##_nn_128x128, et, false) \
+    MAIZE_TILE_BY_LINES(maize_tile_##tag##_nt_128x128, et, true)
 MAIZE_TILE_8(e4m3, 2)
 MAIZE_TILE_8(e5m2, 5)
 MAIZE_TILE_8(e4m3e5m2, 4)
@@ -711,6 +733,7 @@ MAIZE_TILE(maize_tile_f32_nt_128x128, 6, false, true, 128, 128, 2, 2)
 #undef MAIZE_TILE_16
 #undef MAIZE_TILE_8
 #undef MAIZE_TILE_FP
+#undef MAIZE_TILE_BY_LINES
 #undef MAIZE_TILE
 
 }  // namespace maize

@@ -193,5 +193,15 @@ MAIZE_MAP uint32_t we_read(uint32_t es, uint32_t rb, uint32_t cg, uint32_t lane)
     return we_offset(es, rb, (es == 4u ? 4u : 2u) * (lane >> 4), cg * 16u + we_column(es, lane));
 }
 
+// ---- Rows on 128-byte lines -----------------------------------------------------------------------------------------
+// How many K tiles (128 bytes of a row) reach into a second line: 0 none, 1 every other row's (rows on half lines), 2 most.
+// `start`, `pitch`, `stride`: bytes, of the first row, from row to row, from product to product of a batch (0: one product).
+MAIZE_MAP uint32_t off_lines(uint64_t start, uint64_t pitch, uint64_t stride) {
+    return ((start | pitch | stride) & 127u) == 0u ? 0u : ((start | pitch | stride) & 63u) == 0u ? 1u : 2u;
+}
+// Whether 128 x 128 tiles ask for the K tiles of a row in pairs (gemm_tile.hpp), from off_lines of A and B: where half of
+// the rows or more share lines between K tiles.  A row-major B's K tiles are rows of their own and share none.
+MAIZE_MAP bool in_pairs(bool nt, uint32_t a, uint32_t b) { return a + (nt ? b : a) >= 2u; }
+
 }  // namespace maps
 }  // namespace maize

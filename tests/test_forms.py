@@ -78,6 +78,39 @@ def test_the_64_column_tiles_of_a_row_major_b_are_whole_and_free_of_bank_conflic
     assert subprocess.run([str(exe)]).returncode == 0
 
 
+LINES = r"""
+#include "maps.hpp"
+using namespace maize::maps;
+// the K tiles of a row that reach into a second line, in rows of 1024 (none, every other, more)
+static unsigned counted(unsigned long long start, unsigned long long pitch) {
+    unsigned n = 0;
+    for (unsigned r = 0; r < 1024; ++r) n += (start + r * pitch) % 128 != 0;
+    return n == 0 ? 0 : n <= 512 ? 1 : 2;
+}
+int main() {
+    for (unsigned pitch = 1; pitch < 600; ++pitch) if (off_lines(1u << 20, pitch, 0) != counted(1u << 20, pitch)) return 1;
+    for (unsigned start = 1; start < 128; ++start) if (off_lines(start, 256, 0) == 0 || off_lines(0, 256, start) == 0) return 2;
+    if (off_lines(128, 384, 1u << 30) != 0) return 3;
+    // rows on lines: single requests, whatever a row-major B's do; N x K: half of the rows have to share lines
+    for (unsigned b = 0; b < 3; ++b) if (in_pairs(false, 0, b) || !in_pairs(false, 1, b) || !in_pairs(false, 2, b)) return 4;
+    for (unsigned a = 0; a < 3; ++a) for (unsigned b = 0; b < 3; ++b) if (in_pairs(true, a, b) != (a + b >= 2)) return 5;
+    return 0;
+}
+"""
+
+
+def test_tiles_of_128_by_128_ask_in_pairs_only_where_rows_share_lines(tmp_path):
+    """Rows on 128-byte lines have nothing to share, and pairs then cost up to 5 %."""
+    src, exe = tmp_path / "lines.cpp", tmp_path / "lines"
+    src.write_text(LINES)
+    kdir = os.path.join(ROOT, "maize_amd", "csrc", "kernels")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I", kdir, "-o", str(exe), str(src)], check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
+    text = open(os.path.join(kdir, "gemm_tile.hpp")).read()
+    assert "if (maps::in_pairs(NT, off(p.a, lda_of(p), p.stride_a), off(p.b, ldb_of(p), p.stride_b))) body<ET, false, NT, 128, 128, 5, true>(p, lds);" in text
+    assert "else body<ET, false, NT, 128, 128, 4, false>(p, lds);" in text
+
+
 @pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(HSACO)), reason="needs the ROCm llvm-objdump and the built code object")
 def test_form_kernels_keep_to_registers_and_plain_stores():
     text = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", HSACO], check=True, capture_output=True, text=True).stdout

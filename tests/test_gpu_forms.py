@@ -208,9 +208,12 @@ def test_a_captured_form_in_k_ranges_equals_the_eager_one(ctx, warm):
                                      ("e4m3", "64x64w"), ("e4m3", "64x128"), ("e4m3", "128x128")])
 def test_every_count_of_k_tiles(ctx, oracle, forms, op, tile, layout):
     """One K tile to two rounds of the three to five ring stages and a ragged one behind: each count of entries that the requests
-    (one by one or in pairs), the one without a partner and the stage of the tail can meet."""
+    (one by one or in pairs), the one without a partner and the stage of the tail can meet.  128 x 128: with every row on a
+    128-byte line (single requests) and with none there (pairs)."""
     bm, bn = TILES[tile]
     kt = 64 if op == "bf16" else 128
     for entries in range(1, 13):
         for more in (0, 9):
-            check_form(ctx, oracle, forms, op, tile, layout, bm - 3, bn + 5, entries * kt + more, off=entries % 2, pad=more % 2)
+            k = entries * kt + more
+            for lines in (True, False) if tile == "128x128" else (False,):
+                check_form(ctx, oracle, forms, op, tile, layout, bm - 3, bn + 5, k, off=0 if lines else entries % 2, pad=-k % kt if lines else 1 - entries % 2 + more % 2)
