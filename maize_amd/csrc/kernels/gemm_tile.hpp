@@ -575,8 +575,10 @@ __device__ __forceinline__ void body(const GemmArgs& p, char* lds_a) {
         step(S0, TWO, s);
         step(S1, TWO, s + 1u);
     }
-    // The last entries, at most NS + 2: one of the first two may still have one to request or the tail to place.
-    drain<0, NS + 2>(s, ns, [&](auto i_, uint32_t e) { step(std::integral_constant<int, decltype(i_)::value & 1>{}, std::integral_constant<int, (decltype(i_)::value < 2)>{}, e); });
+    // The last entries, the tail among them.  Single requests: at most NS + 1 and the tail; one of the first two steps may still have an entry
+    // to request or the tail to place.  Pairs: at most five (up to s + 3 are requested) and the tail; the first step requests
+    // the fifth and places the tail.
+    drain<0, PAIR ? 6 : NS + 2>(s, ns, [&](auto i_, uint32_t e) { step(std::integral_constant<int, decltype(i_)::value & 1>{}, std::integral_constant<int, (decltype(i_)::value < 2)>{}, e); });
     // nothing may land any more, and the last MFMAs have left the pipe (assembly: invisible to the hazard recognizer)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 

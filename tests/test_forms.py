@@ -213,3 +213,25 @@ def test_where_no_form_can_run(in_type):
                 assert mz.gemm_form(describe(40, 50, 60, nt, in_type, **{ld: 1 << 21})) is None
             except mz.MaizeError:                                # (some are refused altogether: there is one fp64 kernel)
                 assert in_type == mz.IN_F64
+
+
+@pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(HSACO)), reason="needs the ROCm llvm-objdump and the built code object")
+def test_no_k_step_is_written_out_that_none_can_reach():
+    """A ring's code: two K steps in the loop and one each for the last entries.  The loop ends with NS + 1 direct entries left, pairs
+    (five stages) with five, and there may be a tail."""
+    text = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", HSACO], check=True, capture_output=True, text=True).stdout
+    found = {}
+    for line in text.splitlines():
+        head = re.match(r"^[0-9a-f]+ <(maize_\w+)>:", line)
+        if head:
+            kernel = head.group(1)
+            found[kernel] = 0
+        elif "\tv_mfma_" in line:
+            found[kernel] += 1
+    for kernel, got in found.items():
+        op, bm, bn, wide = re.fullmatch(r"maize_tile_([a-z0-9]+)_n[nt]_(\d+)x(\d+)(w?)", kernel).groups()
+        if op in ("f32", "f64") or wide:
+            continue
+        step = int(bm) * int(bn) // 1024 * (2 if op in ("bf16", "f16") else 1)         # matrix instructions of a wave in a K tile
+        last = {("32", "128"): [6], ("64", "64"): [7], ("64", "128"): [5], ("128", "128"): [6, 6]}[bm, bn]
+        assert got == step * sum(2 + n for n in last), (kernel, got)
