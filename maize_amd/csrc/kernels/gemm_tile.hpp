@@ -356,7 +356,7 @@ __device__ __forceinline__ void body(const GemmArgs& p, char* lds_a) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = accx4{0, 0, 0, 0};
 
-    // ---- the tail's loads, then the ring's first NS entries ----------------------------------------------------------
+    // ---- the tail's loads, then the ring's first entries: NS, or four in two pairs -------------------------------------
     // (128 x 128 fp32: when they are placed, two workgroups per compute unit leave no registers to hold them through the loop)
     constexpr bool LATE_TAIL = FP && BM * BN > 64 * 128;
     u32x4 ta[PA], tb[PB];
@@ -430,9 +430,13 @@ __device__ __forceinline__ void body(const GemmArgs& p, char* lds_a) {
         for (int j = 0; j < NJ; ++j) b_rd[j] = (uint32_t)(uintptr_t)(lds_ptr)lds_b + KNB::read(wn * NJ + j, lane);
     }
     // ---- the K loop: a K tile's fragments are read whole, while the MFMAs of the one before run ----------------------------
-    // At the top of a step the entry's fragments are in registers (set S) for every wave.  Behind the barrier the next entry
-    // has landed and this one's stage is free: its requests (entry s + NS) and the next entry's reads (set 1 - S) go out
-    // behind the MFMAs.  One LDS round trip per step, with one wave per SIMD to hide it: reading K half by K half -- two round
+    // At the top of step s entry s's fragments are in registers (set S = s % 2) for every wave.  Behind the barrier entry s + 1
+    // has landed and entry s's stage is free: the requests and the reads of entry s + 1 (set 1 - S) go out behind the MFMAs.
+    //   Single requests: step s asks for entry s + NS, into entry s's stage; the wait leaves the entries from s + 2 on in flight.
+    //   Pairs: up to s + 3 is asked for at the top of an even step s, and s + 1 has landed.  It asks for A of s + 4 and s + 5, into the
+    //   stages of s - 1 and s; step s + 1 asks for B of both, and its wait leaves that A (2 PA requests) in flight: s + 2 and s + 3 have landed.
+    //   An entry s + 4 without a partner and the tail behind it are step s's, the first behind the loop.
+    // One LDS round trip per step, with one wave per SIMD to hide it: reading K half by K half -- two round
     // trips -- 256 x 256 x 4096 on 16 workgroups took 17.6 us against 16.7 (and 14.4 with no requests past the end).
     // (The waits name every register the reads fill, so that nothing derived from them can move in front.)
     // 4- and 8-byte operands: a lane's 16-byte chunk (row-major B: its CH rows of one column) feeds CH instructions four deep,
@@ -499,12 +503,12 @@ __device__ __forceinline__ void body(const GemmArgs& p, char* lds_a) {
     };
     uint32_t st = 0u;                                                 // ring stage of the entry in hand
     uint32_t left = 0u;                                               // an entry without a partner is on its way
-    auto step = [&](auto set, auto requests, uint32_t s) {            // 2: requests entry s + NS; 1: if there is one (or places the tail); 0: there is none
+    auto step = [&](auto set, auto requests, uint32_t s) {            // 2: requests as above; 1: if there is an entry left (or places the tail); 0: there is none
         constexpr int S = decltype(set)::value;
         constexpr int REQ = decltype(requests)::value;
         constexpr std::integral_constant<int, 1 - S> other{};
         if constexpr (PAIR) {
-            // entry s + 1 landed with entry s (S = 0), or all but the youngest requests (of A: two entries' ahead of it) have
+            // (an even step's next entry landed with its own: a barrier only, but behind the last requests, where all are waited for)
             if constexpr (S == 0 && REQ != 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             else if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(2 * PA) : "memory");
             else meet(REQ == 1 ? left : 0u);

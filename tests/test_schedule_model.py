@@ -117,7 +117,8 @@ def mt256_wave_program(nk, slots, nt, barrier_eighth=6):
 
 
 def check_two_stage(ops, steps, nreads, parts=4, pieces=16, nst=2):
-    """`nreads`: fragment reads per part of a K step if a number; a list gives, per part, how many reads of the
+    """("write", tile, piece, stage): a piece written to LDS by the wave itself, done at its next barrier.
+    `nreads`: fragment reads per part of a K step if a number; a list gives, per part, how many reads of the
     tile must have been issued before the part's first MFMA (cumulative).  `nst`: ring stages; with more than two a
     barrier may stand with younger requests still in flight (("wait_keep", n) waits for all but the n youngest)."""
     cumulative = [nreads * (q + 1) for q in range(parts)] if isinstance(nreads, int) else list(nreads)
@@ -132,7 +133,7 @@ def check_two_stage(ops, steps, nreads, parts=4, pieces=16, nst=2):
     reads_seen = {}
     consumed = []
     for op in ops:
-        if op[0] == "dma":
+        if op[0] in ("dma", "write"):
             _, tile, pc, stage = op
             if (tile, pc) in dma_epoch:
                 raise Hazard(f"piece {pc} of tile {tile} requested twice")
@@ -146,7 +147,10 @@ def check_two_stage(ops, steps, nreads, parts=4, pieces=16, nst=2):
                 raise Hazard(f"tile {tile} overwrites tile {old} before all of its fragments were read")
             dma_epoch[(tile, pc)] = epoch
             stage_of[tile] = stage
-            pending.append((tile, pc))
+            if op[0] == "dma":
+                pending.append((tile, pc))
+            else:
+                completed.add((tile, pc))
         elif op[0] == "wait_all":
             completed.update(pending)
             pending = []
@@ -901,3 +905,150 @@ def test_skinny_nt_row_group_ring_is_hazard_free(nb, mr):
         check_ring(ops, turns, None, ring)
         with pytest.raises(Hazard):                              # one load more left in flight: block b's last piece may be missing
             check_ring(*skinny_nt_rows_program(32, ring, primed, ahead, wave, mr, slack=1), None, ring)
+
+
+# ---------------------------------------------------------------------------------------
+# the launcher's forms (gemm_tile.hpp): an entry is a K tile of eight pieces (four of A, four of B: 128 x 128 tiles) or, last, the
+# tail, which the wave writes itself.  Single requests (three to five stages): step s asks for entry s + NS.
+# Pairs (five stages): even steps ask for A of s + 4 and s + 5, odd ones for B of them, two steps per turn
+# ---------------------------------------------------------------------------------------
+TILE_LINES = ("constexpr uint32_t PRIME = PAIR ? 4u : (uint32_t)NS;",
+              "for (; s + 1u < primed; s += 2u) request_pair(s, s);\n        if (s < primed) request(s, s);",
+              "const TileReq r = tile_req(s, st), r2 = tile_req(s + 1u, st + 1u);",
+              "if (tail_here && nd < (uint32_t)NS) place_tail(nd);",
+              "if (n == (uint32_t)c) wait_loads<c * P>();",
+              "meet(PAIR ? (primed > 2u ? primed - 2u : 0u) : primed ? primed - 1u : 0u);",
+              'if constexpr (S == 0 && REQ != 0) asm volatile("s_waitcnt lgkmcnt(0)\\n\\ts_barrier" ::: "memory");\n'
+              '            else if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\\n\\ts_barrier" :: "n"(2 * PA) : "memory");\n'
+              "            else meet(REQ == 1 ? left : 0u);",
+              'else if constexpr (REQ == 2) asm volatile("s_waitcnt vmcnt(%0)\\n\\ts_barrier" :: "n"((NS - 2) * P) : "memory");\n'
+              "        else meet(nd < s + 2u ? 0u : nd - s - 2u < (uint32_t)NS - 2u ? nd - s - 2u : (uint32_t)NS - 2u);",
+              "if constexpr (S == 0) { r = tile_req(s + 4u, pst); r2 = tile_req(s + 5u, st); }\n"
+              "            else                  { r = tile_req(s + 3u, pst ? pst - 1u : (uint32_t)NS - 1u); r2 = tile_req(s + 4u, pst); }",
+              "else if constexpr (REQ == 2) r = tile_req(s + (uint32_t)NS, st);",
+              "if (s + 4u < nd) { request(s + 4u, pst); left = 1u; }\n            if (tail_here && nd >= (uint32_t)NS) place_tail(s + 4u < nd ? st : pst);",
+              "if (s + (uint32_t)NS < nd) request(s + (uint32_t)NS, st);\n            else if (tail_here && s + (uint32_t)NS == nd) place_tail(st);",
+              "if constexpr (PAIR) piece(q & 1 ? r2 : r, S * PA + q / 2);",
+              "for (; s + (PAIR ? 5u : (uint32_t)NS + 1u) < nd; s += 2u) {\n        step(S0, TWO, s);\n        step(S1, TWO, s + 1u);",
+              "drain<0, PAIR ? 6 : NS + 2>(s, ns, ", "std::integral_constant<int, (decltype(i_)::value < 2)>{}, e)")
+
+
+def tile_form_program(nd, tail, pair, stages=None, keep=None, even_barrier=True, first_keep=2, loop_margin=None, tail_stage=None, last=None):
+    """One wave's stream for `nd` K tiles and, if `tail`, the tail behind them; the parameters are the schedule's own unless given."""
+    src = open(os.path.join(KDIR, "gemm_tile.hpp")).read()
+    for fact in TILE_LINES:
+        assert fact in src, fact
+    stages, pa, p = stages or (5 if pair else 4), 4, 8
+    total = nd + (1 if tail else 0)
+    keep = (2 * pa if pair else (stages - 2) * p) if keep is None else keep
+    margin = (5 if pair else stages + 1) if loop_margin is None else loop_margin
+    last = (6 if pair else stages + 2) if last is None else last
+    ops = []
+
+    def request(e, st):
+        ops.extend(("dma", e, pc, st) for pc in range(p))
+
+    def place(st):
+        ops.extend(("write", nd, pc, st) for pc in range(p))
+
+    def meet(n):
+        ops.extend([("wait_keep", n * p)] if n < stages else [])
+        ops.append(("barrier",))
+
+    primed = min(nd, 4 if pair else stages)
+    e = 0
+    while pair and e + 1 < primed:
+        for pc in range(p):
+            ops += [("dma", e, pc, e), ("dma", e + 1, pc, e + 1)]
+        e += 2
+    for e in range(e, primed):
+        request(e, e)
+    if tail and nd < stages:
+        place(nd)
+    meet((max(primed - first_keep, 0) if pair else max(primed - 1, 0)))
+    ops += [("read", 0, 0, 0)] * 16
+    st, left = 0, 0
+
+    def step(even, req, s):
+        nonlocal st, left
+        if pair:
+            if even and req:
+                ops.extend([("barrier",)] if even_barrier else [])
+            elif req == 2:
+                ops.extend([("wait_keep", keep), ("barrier",)])
+            else:
+                meet(left if req == 1 else 0)
+        elif req == 2:
+            ops.extend([("wait_keep", keep), ("barrier",)])
+        else:
+            meet(0 if nd < s + 2 else min(nd - s - 2, stages - 2))
+        pst = st - 1 if st else stages - 1
+        out = []
+        if req == 2 and pair:
+            r, r2 = ((s + 4, pst), (s + 5, st)) if even else ((s + 3, pst - 1 if pst else stages - 1), (s + 4, pst))
+            out = [("dma", (r2 if q & 1 else r)[0], (0 if even else pa) + q // 2, (r2 if q & 1 else r)[1]) for q in range(8)]
+        elif req == 2:
+            out = [("dma", s + stages, pc, st) for pc in range(p)]
+        elif req == 1 and pair and even:
+            if s + 4 < nd:
+                request(s + 4, pst)
+                left = 1
+            if tail and nd >= stages:
+                place((st if s + 4 < nd else pst) if tail_stage is None else tail_stage(st, pst))
+        elif req == 1 and not pair:
+            if s + stages < nd:
+                request(s + stages, st)
+            elif tail and s + stages == nd:
+                place(st)
+        nst = (st + 1) % stages
+        for m in range(16):
+            ops.append(("mfma", s, 0))
+            if s + 1 < total:                                # (a read past the last entry brings in what nothing multiplies)
+                ops.append(("read", s + 1, 0, nst))
+            if m % 2 == 0 and out:
+                ops.append(out[m // 2])
+        st = nst
+
+    s = 0
+    while s + margin < nd:
+        step(True, 2, s)
+        step(False, 2, s + 1)
+        s += 2
+    for i in range(last):
+        if s < total:
+            step(i % 2 == 0, 1 if i < 2 else 0, s)
+            s += 1
+    ops.append(("wait_all",))
+    return ops, total
+
+
+TILE_ENTRIES = [(nd, tail) for nd in range(34) for tail in (False, True) if nd or tail]
+
+
+@pytest.mark.parametrize("pair,stages", [(False, 3), (False, 4), (False, 5), (True, 5)])
+def test_form_rings_are_hazard_free(pair, stages):
+    for nd, tail in TILE_ENTRIES:
+        ops, total = tile_form_program(nd, tail, pair, stages)
+        assert check_two_stage(ops, total, 16, parts=1, pieces=8, nst=stages) == total - 1, (nd, tail)
+
+
+@pytest.mark.parametrize("why,pair,change", [
+    ("a request more in flight at an odd step", True, dict(keep=9)),
+    ("a request more in flight at a step", False, dict(keep=17)),
+    ("no barrier at an even step: s + 5 goes into the stage that other waves still read", True, dict(even_barrier=False)),
+    ("entry 1 not waited for in front of the first step", True, dict(first_keep=1)),
+    ("pairs up to an entry that is not there", True, dict(loop_margin=4)),
+    ("the tail always where an entry without a partner leaves it", True, dict(tail_stage=lambda st, pst: st)),
+    ("the tail always in the stage of the entry before", True, dict(tail_stage=lambda st, pst: pst)),
+    ("one step too few behind the loop", True, dict(last=5)),
+    ("one step too few behind the loop", False, dict(last=5)),
+])
+def test_form_ring_checker_rejects_broken_schedules(why, pair, change):
+    def broken(nd, tail):
+        try:
+            ops, total = tile_form_program(nd, tail, pair, **change)
+            return check_two_stage(ops, total, 16, parts=1, pieces=8, nst=5 if pair else 4) != total - 1
+        except Hazard:
+            return True
+
+    assert any(broken(nd, tail) for nd, tail in TILE_ENTRIES), why
