@@ -211,9 +211,14 @@ def test_every_count_of_k_tiles(ctx, oracle, forms, op, tile, layout):
     (one by one or in pairs), the one without a partner and the stage of the tail can meet.  128 x 128: with every row on a
     128-byte line (single requests) and with none there (pairs)."""
     bm, bn = TILES[tile]
-    kt = 64 if op == "bf16" else 128
+    kt, es = (64, 2) if op == "bf16" else (128, 1)
+    met = set()
     for entries in range(1, 13):
-        for more in (0, 9):
+        # (a row-major B whose rows are no whole dwords makes its last whole K tile a tail: bn + 5 columns, but not bn + 4)
+        for more, n in ((0, bn + 4), (9, bn + 5)) + (((0, bn + 5),) if layout == NN else ()):
             k = entries * kt + more
+            tail = k % kt != 0 or (layout == NN and n * es % 4 != 0)
+            met.add((entries - (1 if tail and not more else 0), tail))
             for lines in (True, False) if tile == "128x128" else (False,):
-                check_form(ctx, oracle, forms, op, tile, layout, bm - 3, bn + 5, k, off=0 if lines else entries % 2, pad=-k % kt if lines else 1 - entries % 2 + more % 2)
+                check_form(ctx, oracle, forms, op, tile, layout, bm - 3, n, k, off=0 if lines else entries % 2, pad=-k % kt if lines else 1 - entries % 2 + more % 2)
+    assert met >= {(nd, tail) for nd in range(1, 13) for tail in (False, True)}, met        # by direct loads, and whether a tail follows
