@@ -107,8 +107,8 @@ def test_tiles_of_128_by_128_ask_in_pairs_only_where_rows_share_lines(tmp_path):
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", kdir, "-o", str(exe), str(src)], check=True)
     assert subprocess.run([str(exe)]).returncode == 0
     text = open(os.path.join(kdir, "gemm_tile.hpp")).read()
-    assert "if (maps::in_pairs(NT, off(p.a, lda_of(p), p.stride_a), off(p.b, ldb_of(p), p.stride_b))) body<ET, false, NT, 128, 128, 5, true>(p, lds);" in text
-    assert "else body<ET, false, NT, 128, 128, 4, false>(p, lds);" in text
+    assert "const bool pairs = BY_LINES && maps::in_pairs(NT, off(p.a, lda, p.stride_a), off(p.b, ldb, p.stride_b));" in text
+    assert re.search(r"\} else if \(pairs\) \{\s+constexpr bool PAIR = true;\s+constexpr int NS = RING;\s+#include \"gemm_tile_ring.hpp\"\s+\} else \{\s+constexpr bool PAIR = false;", text)
 
 
 @pytest.mark.skipif(not (os.path.exists(OBJDUMP) and os.path.exists(HSACO)), reason="needs the ROCm llvm-objdump and the built code object")

@@ -908,11 +908,11 @@ def test_skinny_nt_row_group_ring_is_hazard_free(nb, mr):
 
 
 # ---------------------------------------------------------------------------------------
-# the launcher's forms (gemm_tile.hpp): an entry is a K tile of eight pieces (four of A, four of B: 128 x 128 tiles) or, last, the
+# the launcher's forms (gemm_tile.hpp, gemm_tile_ring.hpp): an entry is a K tile of eight pieces (four of A, four of B: 128 x 128 tiles) or, last, the
 # tail, which the wave writes itself.  Single requests (three to five stages): step s asks for entry s + NS.
 # Pairs (five stages): even steps ask for A of s + 4 and s + 5, odd ones for B of them, two steps per turn
 # ---------------------------------------------------------------------------------------
-TILE_LINES = ("constexpr uint32_t PRIME = PAIR ? 4u : (uint32_t)NS;",
+TILE_LINES = ("constexpr bool PAIR = false;\n        constexpr int NS = RING - 1;", "constexpr uint32_t PRIME = PAIR ? 4u : (uint32_t)NS;",
               "for (; s + 1u < primed; s += 2u) request_pair(s, s);\n        if (s < primed) request(s, s);",
               "const TileReq r = tile_req(s, st), r2 = tile_req(s + 1u, st + 1u);",
               "if (tail_here && nd < (uint32_t)NS) place_tail(nd);",
@@ -935,7 +935,7 @@ TILE_LINES = ("constexpr uint32_t PRIME = PAIR ? 4u : (uint32_t)NS;",
 
 def tile_form_program(nd, tail, pair, stages=None, keep=None, even_barrier=True, first_keep=2, loop_margin=None, tail_stage=None, last=None):
     """One wave's stream for `nd` K tiles and, if `tail`, the tail behind them; the parameters are the schedule's own unless given."""
-    src = open(os.path.join(KDIR, "gemm_tile.hpp")).read()
+    src = open(os.path.join(KDIR, "gemm_tile.hpp")).read() + open(os.path.join(KDIR, "gemm_tile_ring.hpp")).read()
     for fact in TILE_LINES:
         assert fact in src, fact
     stages, pa, p = stages or (5 if pair else 4), 4, 8
