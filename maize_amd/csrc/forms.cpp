@@ -47,7 +47,8 @@ const Names& names() {
 struct TileCost { uint32_t bm, bn; double t0, one, many, turn, r0, r1, ua, ub, nn, bw, tail, e8; };
 // 128 x 128 has a compute unit to itself and half of the LDS fill per product of 64 x 128: where its tiles make up one round or
 // few (129 to 256: 1024 x 3072 x 1999 into bf16 30.1 -> 24.5 us, 4499 x 520 x 3644 51.1 -> 35.8; below, K ranges of smaller tiles
-// keep the chip busier).  Fitted to 110 timings, residuals 7 % where it is a candidate.
+// keep the chip busier).  Fitted to 110 timings of single requests, residuals 7 % where it is a candidate; products whose rows lie off
+// 128-byte lines run on requests in pairs now (gemm_tile.hpp), 5 % faster on average and up to 22, for which there is no term.
 constexpr TileCost kTileCost[kTiles] = {
     {32, 128, 3.62, 0.215, 0.371, 0.0, 1.63, 0.14, 0.18, 0.36, 0.0, 6.55, 0.55, 0.07},
     {64, 64, 3.97, 0.167, 0.177, 1.06, 1.82, 0.19, 0.11, 0.40, 0.14, 6.88, 0.30, 0.10},
@@ -223,7 +224,8 @@ bool choose_form(const maize_gemm_ex_desc_t& d, uint32_t registry, uint32_t comp
             if (ks > 1u && (tiles * ks > (pinned ? 8u : 2u) * compute_units || p.steps / ks < 3u || t == T128x128)) break;
             if (ks > 1u && cdiv(p.steps, cdiv(p.steps, ks)) != ks) continue;
             // (16- and 8-bit 128 x 128: from ten K tiles on and 8 % ahead of the others by the model: of 220 products 20 then run on it,
-            // 1.19x on average, one of them 3 % slower; without the two conditions up to 30 % slower, 413 deep)
+            // 1.19x on average, one of them 3 % slower; without the two conditions up to 30 % slower, 413 deep.  Measured, as the row of
+            // kTileCost, with single requests throughout)
             const bool big = t == T128x128 && fam != kWide;
             if (big && p.steps < 10u) break;
             const double cost = tile_cost(c, p, tiles, ks);

@@ -29,8 +29,8 @@
 // 128 x 168 x 296 63 -> 5.5.  (Tried and slower: twice the ring depth on one workgroup per compute unit, three stages on three.)
 //
 // 128 x 128 of 16- and 8-bit operands: what bounds the smaller tiles on a product of a round or two is the LDS fill, which this
-// halves per multiply-add.  What bounds it in turn is one wave per SIMD (1024 x 3072 x 1999: waits 0.30, waits to issue 0.35, matrix pipe
-// 0.30).  One workgroup of five ring stages (the 160 KiB) per compute unit: two of two stages have too few
+// halves per multiply-add.  What bounds it in turn is one wave per SIMD (1024 x 3072 x 1999 into fp32: waits 0.32, waits to issue 0.31,
+// matrix pipe 0.31).  One workgroup of four or five ring stages (of 160 KiB) per compute unit: two of two stages have too few
 // registers, and the compiler then copies fragments that are still being read.  1024 x 3072 x 1999 accumulated into fp32
 // 29.6 -> 25.3 us (424 -> 496 TFLOP/s), 3713 x 554 x 4707 in batches of 3 200 -> 140, E4M3 928 x 2568 x 5992 42.6 -> 32.9.
 //
@@ -40,9 +40,9 @@
 // 1856 (rows on lines) 1.474 both.  Single requests from four stages -> pairs: 1700 x 2000 x 4999 57.1 -> 52.0 us (595 ->
 // 654 TFLOP/s), E4M3 928 x 2568 x 5992 35.4 -> 29.1, 1024 x 3072 x 1999 K x N into fp32 25.4 -> 24.6, 96 drawn products 5 % off on
 // average and none longer.  Rows that do not start on dwords gain nothing (E4M3 1024 x 3072 x 1999 N x K 21.3 both): a request there is
-// about four accesses of the vector cache, which then bound the loop.
+// about four accesses of the vector cache, and pairs leave their number as it is (22.0 million; L2 reads 1.65 -> 1.31).
 // Rows on lines share nothing, and B is asked for one step later: 32 drawn products 2 % longer on average, 7 % at most (1192 x
-// 2580 x 1856 N x K 18.1 -> 19.1, E5M2 5176 x 2006 x 4096 51.2 -> 53.8, 1536 x 2203 x 4096 K x N 36.9 -> 38.5).  They have single requests and
+// 2580 x 1856 N x K 18.1 -> 19.1, E5M2 5176 x 2006 x 4096 51.2 -> 53.8, 1536 x 2203 x 4096 K x N 36.9 -> 38.2).  They have single requests and
 // four stages (with five, a K tile more stands in front of the first multiplication: 1 to 5 % longer as well); so have N x K products with one
 // operand on lines and one on half lines, which gain and lose 4 %.  One operand on lines and one anywhere: 1 to 5 % off on average, 2 %
 // longer at most; both on half lines, or A against a row-major B: 3 % off, 3 % longer at most.  The kernel looks at its operands
